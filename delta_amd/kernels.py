@@ -758,6 +758,67 @@ def gemm_rows32_silu(x: torch.Tensor, w13: torch.Tensor, out: Optional[torch.Ten
     return out
 
 
+def gemm_rows128_ok(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """True when ``delta_gemm_rows128`` takes ``x @ weight.T`` for an inference call: at most 128
+    contiguous, 16-byte aligned rows of a bf16/fp16 weight of x's dtype, K % 64 == 0, N % 16 == 0."""
+    if x.dtype not in _DTYPES or weight.dtype != x.dtype or weight.dim() != 2 or not x.is_cuda \
+            or weight.device != x.device:
+        return False
+    if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+        return False
+    N, Kd = weight.shape
+    rows = x.numel() // max(x.shape[-1], 1)
+    return (x.shape[-1] == Kd and Kd % 64 == 0 and N % 16 == 0 and 0 < rows <= 128 and x.is_contiguous()
+            and x.data_ptr() % 16 == 0 and Kd <= 1 << 23 and weight.stride(1) == 1 and weight.stride(0) >= Kd
+            and weight.stride(0) % 8 == 0 and weight.data_ptr() % 16 == 0 and (N + 192) * weight.stride(0) < 1 << 31)
+
+
+def gemm_rows128_splits(M: int, N: int, K: int) -> int:
+    """K splits ``delta_gemm_rows128`` uses for this shape (1: rounded output; > 1: fp32 partials)."""
+    return int(_lib.query("delta_gemm_rows128_splits", int(M), int(N), int(K)))
+
+
+def gemm_rows128(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                 out: Optional[torch.Tensor] = None, partials: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """``x @ weight.T (+ bias)`` for <= 128 token rows on ``delta_gemm_rows128``; returns as
+    ``gemm_rows32`` does: the rounded output ``[..., N]``, or the fp32 partials ``[S, M, N]``."""
+    dev = _check_cuda(x, weight, bias, out, partials)
+    N, Kd = weight.shape
+    if x.shape[-1] != Kd:
+        raise ValueError(f"x has {x.shape[-1]} features, weight expects {Kd}")
+    if weight.dtype != x.dtype or (bias is not None and (bias.dtype != x.dtype or bias.numel() != N
+                                                         or not bias.is_contiguous())):
+        raise TypeError("x, weight and bias must share a dtype; bias must be contiguous [N]")
+    if weight.stride(1) != 1:
+        raise ValueError("weight rows must be contiguous")
+    x2 = _rows2d("x", x, Kd)
+    M = x2.shape[0]
+    S = gemm_rows128_splits(M, N, Kd)
+    if S < 1:
+        raise ValueError(f"delta_gemm_rows128 does not take [{M}, {Kd}] x [{N}, {Kd}]^T")
+    o2 = None
+    if S == 1:
+        if out is None:
+            out = torch.empty(*x.shape[:-1], N, dtype=x.dtype, device=dev)
+        o2 = out.reshape(-1, N)
+        if o2.stride(1) != 1 or o2.shape[0] != M or o2.data_ptr() != out.data_ptr() or o2.dtype != x.dtype:
+            raise ValueError("out must be [..., N] of x's dtype with contiguous rows")
+    else:
+        if partials is None:
+            partials = torch.empty(S, M, N, dtype=torch.float32, device=dev)
+        if partials.dtype != torch.float32 or not partials.is_contiguous() or tuple(partials.shape) != (S, M, N):
+            raise ValueError(f"partials must be contiguous fp32 [{S}, {M}, {N}]")
+    _lib.call("delta_gemm_rows128", x2.data_ptr(), x2.stride(0), weight.data_ptr(), weight.stride(0), _ptr(bias),
+              o2.data_ptr() if o2 is not None else None, o2.stride(0) if o2 is not None else 0,
+              partials.data_ptr() if S > 1 else None, int(M), int(N), int(Kd), _dtype_code(x), _stream(dev))
+    return out if S == 1 else partials
+
+
+def gemm_rows128_silu(x: torch.Tensor, w13: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """The fused gate/up GEMM + SiLU-mul for <= 128 token rows (``delta_gemm_rows128_silu``)."""
+    return gemm_rows32_silu(x, w13, out, _entry="delta_gemm_rows128_silu")
+
+
 def gemm_skinny_silu(x: torch.Tensor, w13: torch.Tensor, out: Optional[torch.Tensor] = None) -> torch.Tensor:
     """The same fused gate/up GEMM + SiLU-mul for <= 8 token rows (``delta_gemm_skinny_silu``)."""
     return gemm_rows32_silu(x, w13, out, _entry="delta_gemm_skinny_silu")

@@ -228,6 +228,17 @@ def dense(x: Tensor, layer: nn.Linear) -> Tensor:
 # that sums partials, the same time for w1|w3).
 _ROWS32_MAX = 32
 
+# At 33-128 token rows the same projections, and the merged w1|w3 with SiLU-mul, go to
+# delta_gemm_rows128 (us, against hipBLASLt; 64 rows: DeepSeek-R1-Distill-Qwen-1.5B w2 9.8 vs 25.4, wo
+# 4.9 vs 7.5, w1|w3 18.2 vs 18.7 and a 5 us SiLU-mul; 128 rows: Qwen2.5-14B w2 34.9 vs 73.9, wo 18.9 vs
+# 32.1, w1|w3 65-73 vs 73 and 5).  It stays on hipBLASLt where that is faster: past 64 rows weights of
+# fewer than 8 M elements (the 1.5B wo: 8.5 vs 7.1, and the norm's partials come on top) and gate/up
+# launches of more than 256 blocks of 64 columns, a second pass over the CUs (Qwen2.5-7B w1|w3: 80-89
+# vs 72); wqkv and lm_head too, whose consumers sum no partials (14B wqkv unsplit 40 vs 33).
+_ROWS128_MAX = 128
+_ROWS128_MIN_WEIGHT = 8 << 20
+_ROWS128_GLU_MAX = 64 * 256
+
 
 def dense_to_norm(x: Tensor, layer: nn.Linear):
     """``layer(x)`` for a consumer that is ``K.add_rmsnorm``: the output, or the fp32 partials
@@ -236,6 +247,10 @@ def dense_to_norm(x: Tensor, layer: nn.Linear):
     rows = x.numel() // x.shape[-1]
     if rows > _SKINNY_ROWS_ANY and rows <= _ROWS32_MAX and K.gemm_skinny_ok(x, w) and w.shape[0] % 64 == 0:
         r = K.gemm_rows32(x, w, layer.bias)
+        return r if r.dtype == torch.float32 else r.view(*x.shape[:-1], w.shape[0])
+    if _ROWS32_MAX < rows <= _ROWS128_MAX and K.gemm_rows128_ok(x, w) \
+            and (rows <= 64 or w.numel() >= _ROWS128_MIN_WEIGHT):
+        r = K.gemm_rows128(x, w, layer.bias)
         return r if r.dtype == torch.float32 else r.view(*x.shape[:-1], w.shape[0])
     return dense(x, layer)
 
@@ -331,10 +346,10 @@ class FeedForward(nn.Module):
     """SwiGLU FFN.  ``w1`` and ``w3`` live in one weight stored transposed, ``w13_t``
     ``[dim, 2 * inter]``, so the gate and up projections are one GEMM ``x @ w13_t``: at
     32-row decode batches hipBLASLt streams this layout at ~5.2 TB/s against ~4.4 TB/s for
-    ``x @ w13.T``.  An engine set up for at most 32 rows per step re-lays it out row-major
+    ``x @ w13.T``.  An engine set up for at most 128 rows per step re-lays it out row-major
     (``w13`` ``[2 * inter, dim]``, ``use_row_major_w13``): ``delta_gemm_skinny`` streams it faster
-    still at <= 8 rows (Qwen2.5-7B, 4 rows: 41 vs 53 us) and ``delta_gemm_rows32_silu`` fuses the
-    SiLU-mul into the GEMM at 9-32 rows.  Checkpoints with separate ``w1`` /
+    still at <= 8 rows (Qwen2.5-7B, 4 rows: 41 vs 53 us) and ``delta_gemm_rows32_silu`` /
+    ``delta_gemm_rows128_silu`` fuse the SiLU-mul into the GEMM at 9-32 and 33-128 rows.  Checkpoints with separate ``w1`` /
     ``w3`` (the reference's names, ``[inter, dim]`` each) are merged and transposed on load."""
 
     def __init__(self, config: ModelArgs) -> None:
@@ -382,6 +397,9 @@ class FeedForward(nn.Module):
                 return dense_to_norm(K.gemm_skinny_silu(x, self.w13), self.w2)
             if rows <= _ROWS32_MAX:
                 return dense_to_norm(K.gemm_rows32_silu(x, self.w13), self.w2)
+        if hasattr(self, "w13") and _ROWS32_MAX < rows <= _ROWS128_MAX and self.inter % 16 == 0 \
+                and (rows <= 64 or self.inter <= _ROWS128_GLU_MAX) and K.gemm_rows128_ok(x, self.w13):
+            return dense_to_norm(K.gemm_rows128_silu(x, self.w13), self.w2)
         return dense_to_norm(K.silu_mul(self._gate_up(x)), self.w2)
 
 

@@ -493,6 +493,21 @@ int delta_gemm_rows32_silu(const void *x, int64_t ldx, const void *w13, int64_t 
 int delta_gemm_skinny_silu(const void *x, int64_t ldx, const void *w13, int64_t ldw, void *out, int64_t ldo,
                            int M, int inter, int K, int dtype, delta_stream_t stream);
 
+/* The decode projections at 33-128 token rows (any M <= 128 is taken): as delta_gemm_rows32, with
+ * delta_gemm_rows128_splits(M, N, K) == 1: out [M, N] (row stride ldo, 8-byte aligned rows) =
+ * dtype(x w^T + bias); S > 1: fp32 partials [S][M][N] (contiguous, 16-byte aligned; bias in split 0
+ * only) for delta_add_rmsnorm_partials, out unused.  S is 1, 2, 4, 8 or 16 and depends only on the
+ * shape; 0 = not taken.  K % 64 == 0, N % 16 == 0, x and w rows 16-byte aligned. */
+int delta_gemm_rows128_splits(int M, int N, int K);
+int delta_gemm_rows128(const void *x, int64_t ldx, const void *w, int64_t ldw, const void *bias, void *out,
+                       int64_t ldo, float *partials, int M, int N, int K, int dtype, delta_stream_t stream);
+
+/* FeedForward's gate/up projections and SiLU-mul in one launch for M <= 128 rows, the roundings of
+ * delta_gemm_rows32_silu: w13 [2 * inter, K] row-major, out [M, inter] with 8-byte aligned rows.
+ * inter % 16 == 0, K % 64 == 0, x and w13 rows 16-byte aligned. */
+int delta_gemm_rows128_silu(const void *x, int64_t ldx, const void *w13, int64_t ldw, void *out, int64_t ldo,
+                            int M, int inter, int K, int dtype, delta_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif
