@@ -44,6 +44,10 @@ SIGNATURES = {
     "delta_paged_prefill": (c_int, [
         _P, c_int64, c_int64, _P, c_int64, _P, _P, _P, c_int64, _P, _P, c_int64, c_int64, _P,
         c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P]),
+    "delta_paged_prefill_rows_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int64]),
+    "delta_paged_prefill_rows": (c_int, [
+        _P, c_int64, c_int64, _P, c_int64, _P, _P, _P, c_int64, _P, _P, c_int64, c_int64, _P,
+        c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, c_size_t, _P]),
     "delta_paged_decode": (c_int, [
         _P, c_int64, c_int64,                 # q, strides
         _P, c_int64,                          # kv_cache, num_pages

@@ -45,6 +45,24 @@ __device__ __forceinline__ u32x4 ld128_stream(const void *p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(p));
 }
 
+// 1 KiB from global memory straight into LDS: lane l's 16 bytes at base + off land at lds + 16 l.
+// Asynchronous (vmcnt, in order with the wave's other loads); the compiler does not see the LDS write,
+// so the caller waits (wait_loads) and fences.  STREAM: nontemporal, for data read once.
+template <bool STREAM = false>
+__device__ __forceinline__ void load_lds_1k(uint32_t lds, const void *base, uint32_t off) {
+  if constexpr (STREAM)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(off), "s"(base)
+                 : "memory");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
+                 : "memory");
+}
+// At most N of the wave's vector loads outstanding, and its LDS reads done.
+template <int N>
+__device__ __forceinline__ void wait_loads() {
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
+}
+
 // Element conversions for a packed 32-bit pair of 16-bit floats.
 template <int DT>
 struct Elem;

@@ -56,6 +56,7 @@ struct DecodeArgs {
   const int32_t *kv_indices;
   int64_t kv_indices_len;
   const int32_t *last_page_len;
+  const int32_t *q_rows;  // ROWS launches: query-token CSR; only rows of exactly one token take part
   uint16_t *o;
   int64_t o_stride_b, o_stride_h;
   float *lse;
@@ -148,7 +149,10 @@ typedef __attribute__((address_space(3))) s4_t lds_s4_t;
 // Work units of a split launch: row b has units_of(b) = clamp(ceil(pages_b / chunk), 1,
 // nsplit) of them (its last unit takes any pages past units * chunk, so a row longer than the
 // planned maximum is still covered), numbered row by row.
+// (ROWS: a row of another token count has one unit, which exits.)
+template <bool ROWS = false>
 __device__ __forceinline__ int units_of(const DecodeArgs &a, int b) {
+  if (ROWS && a.q_rows[b + 1] - a.q_rows[b] != 1) return 1;
   const RowInfo r = row_info(a, b);
   const int n = (r.np + a.chunk - 1) / a.chunk;
   return n < 1 ? 1 : (n > a.nsplit ? a.nsplit : n);
@@ -211,11 +215,12 @@ __device__ int balanced_row(const DecodeArgs &a, int y, int *lds, RowInfo *ri) {
 // the plan), row b at F + b, F = the number of full units.  Blocks start in grid order, so the
 // short last units of a ragged batch fill the launch's tail instead of whole units of the last
 // rows.  A running inclusive scan over 64 rows at a time; false past the last unit.
+template <bool ROWS = false>
 __device__ __forceinline__ bool find_unit(const DecodeArgs &a, int u, int lane, int *row, int *split, int *nu) {
   int base = 0;
   for (int r0 = 0; r0 < a.batch; r0 += 64) {
     const int r = r0 + lane;
-    const int n = r < a.batch ? units_of(a, r) - 1 : 0;  // full units of row r
+    const int n = r < a.batch ? units_of<ROWS>(a, r) - 1 : 0;  // full units of row r
     int incl = n;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -237,7 +242,7 @@ __device__ __forceinline__ bool find_unit(const DecodeArgs &a, int u, int lane, 
   const int b = u - base;  // the last units, one per row
   if (b >= a.batch) return false;
   *row = b;
-  *nu = units_of(a, b);
+  *nu = units_of<ROWS>(a, b);
   *split = *nu - 1;
   return true;
 }
@@ -325,7 +330,8 @@ __device__ __forceinline__ void part_store(float *p, float v) {
     *p = v;
 }
 
-template <int DT, int G, bool WITH_V, bool WITH_DUMP, bool ROPE, bool TOKMAX = false, bool AGENT_PARTS = false>
+template <int DT, int G, bool WITH_V, bool WITH_DUMP, bool ROPE, bool TOKMAX = false, bool AGENT_PARTS = false,
+          bool ROWS = false>
 __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *smem) {
   // No FMA contraction: every instantiation (with or without the dump) rounds the softmax
   // arguments identically, so P -- rounded to the KV dtype for the P.V MFMA -- is the same.
@@ -362,7 +368,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
       nu = nu < 1 ? 1 : (nu > a.nsplit ? a.nsplit : nu);
       if (split >= nu) return;  // whole block
     } else {
-      if (!find_unit(a, unit, lane, &b, &split, &nu)) return;  // past the last unit: whole block
+      if (!find_unit<ROWS>(a, unit, lane, &b, &split, &nu)) return;  // past the last unit: whole block
       ri = row_info(a, b);
     }
     j0 = split * a.chunk;
@@ -375,6 +381,11 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
       ri = row_info(a, b);
     }
     j1 = ri.np;
+  }
+  int qrow = b;  // the row's query token
+  if (ROWS) {
+    qrow = a.q_rows[b];
+    if (a.q_rows[b + 1] - qrow != 1) return;  // whole block
   }
   // A split launch's partial slot (row, split), and whether this is the row's first split;
   // both wave-uniform, so kept in scalar registers across the page loop.
@@ -395,7 +406,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
   // at d = 64 sp + 32 (t / 8) + 8c + [0, 8); zero for heads past the group.
   u32x4 qf[2];
   if ((t & 7) < G) {
-    const uint16_t *qp = a.q + (int64_t)b * a.q_stride_b + (int64_t)(h * G + (t & 7)) * a.q_stride_h +
+    const uint16_t *qp = a.q + (int64_t)qrow * a.q_stride_b + (int64_t)(h * G + (t & 7)) * a.q_stride_h +
                          32 * (t >> 3) + 8 * c;
     qf[0] = ld128(qp);
     qf[1] = ld128(qp + 64);
@@ -966,6 +977,12 @@ __global__ void __launch_bounds__(kMaxWaves * 64) paged_decode_full_kernel(Decod
   extern __shared__ float smem[];
   decode_split_body<DT, G, true, false, ROPE>(a, smem);
 }
+// The rows of one query token of a prompt step (always split: the merge kernel writes o and lse).
+template <int DT, int G>
+__global__ void __launch_bounds__(kMaxWaves * 64) paged_decode_rows_kernel(DecodeArgs a) {
+  extern __shared__ float smem[];
+  decode_split_body<DT, G, true, false, false, false, false, true>(a, smem);
+}
 template <int DT, int G, bool ROPE>
 __global__ void __launch_bounds__(kMaxWaves * 64) paged_decode_subset_kernel(DecodeArgs a) {
   extern __shared__ float smem[];
@@ -1001,7 +1018,7 @@ __global__ void __launch_bounds__(kMaxWaves * 64) paged_decode_plan_tokmax_kerne
 // groups' sums then combine through LDS, so up to 64 splits cost one round of loads.  Partials
 // sit at (row, split), so each group's first batch issues its loads with the row bounds, not
 // after them (splits the row does not have weigh nothing).
-template <int DT>
+template <int DT, bool ROWS>
 __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(DecodeArgs a, int G) {
   using E = Elem<DT>;
   __shared__ float s_m[kMergeGroups], s_l[kMergeGroups], s_a[kMergeGroups][kHeadDim];
@@ -1011,6 +1028,11 @@ __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(D
   const int dd = threadIdx.x % kHeadDim;
   const int grp = threadIdx.x / kHeadDim;
   const int ngrp = blockDim.x / kHeadDim;
+  int orow = b;
+  if (ROWS) {
+    orow = a.q_rows[b];
+    if (a.q_rows[b + 1] - orow != 1) return;  // whole block
+  }
   const int nu = units_of(a, b);
   const int64_t stride = (int64_t)a.hkv * G;  // partial rows per split
   const int64_t p0 = ((int64_t)b * a.nsplit * a.hkv + h) * G + g;
@@ -1068,8 +1090,8 @@ __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(D
     }
     M = MM;
   }
-  a.o[(int64_t)b * a.o_stride_b + (int64_t)hq * a.o_stride_h + dd] = (uint16_t)E::from_float(L > 0.f ? A / L : 0.f);
-  if (dd == 0 && a.lse != nullptr) a.lse[(int64_t)b * a.hq + hq] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
+  a.o[(int64_t)orow * a.o_stride_b + (int64_t)hq * a.o_stride_h + dd] = (uint16_t)E::from_float(L > 0.f ? A / L : 0.f);
+  if (dd == 0 && a.lse != nullptr) a.lse[(int64_t)orow * a.hq + hq] = L > 0.f ? (M + log2f(L)) * kLn2 : -INFINITY;
 }
 
 // lse-only merge (scorer path without V): one 64-lane wave per (row, q head), lanes over units.
@@ -1365,6 +1387,7 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h, const void
   a.kv_indices = kv_indices;
   a.kv_indices_len = kv_indices_len;
   a.last_page_len = kv_last_page_len;
+  a.q_rows = nullptr;
   a.o = (uint16_t *)o;
   a.o_stride_b = o_stride_b;
   a.o_stride_h = o_stride_h;
@@ -1461,15 +1484,98 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h, const void
   if (rc || a.nsplit == 1) return rc;
   if (with_acc) {
     if (dtype == DELTA_BF16)
-      hipLaunchKernelGGL(decode_merge_kernel<DELTA_BF16>, dim3(batch * hq), dim3(kHeadDim * merge_groups(a.nsplit)), 0,
+      hipLaunchKernelGGL((decode_merge_kernel<DELTA_BF16, false>), dim3(batch * hq), dim3(kHeadDim * merge_groups(a.nsplit)), 0,
                          stream, a, G);
     else
-      hipLaunchKernelGGL(decode_merge_kernel<DELTA_FP16>, dim3(batch * hq), dim3(kHeadDim * merge_groups(a.nsplit)), 0,
+      hipLaunchKernelGGL((decode_merge_kernel<DELTA_FP16, false>), dim3(batch * hq), dim3(kHeadDim * merge_groups(a.nsplit)), 0,
                          stream, a, G);
   } else {
     const int n = batch * hq;
     hipLaunchKernelGGL(decode_merge_lse_kernel, dim3((n + 3) / 4), dim3(256), 0, stream, a, G);
   }
+  return check_launch(who);
+}
+
+// The rows of exactly one query token of a prompt step (delta_paged_prefill_rows): decode attention of
+// those rows over packed head-major work units of 4-wave blocks, then the merge.  Row lengths are only
+// on the device; the host knows the pages of all rows together, so a unit holds what brings the launch to
+// about 1024 blocks, 16-128 pages (4-32 per wave), and a row has at most as many units as keep the
+// partials within 2048 (row, unit) slots (8 per row for more than 256 rows; a longer row's last unit
+// takes the rest).
+void decode_rows_plan(int batch, int hkv, int64_t pages, int *nsplit, int *chunk) {
+  int64_t ch = ceil_div(pages * hkv, 1024);
+  ch = ch < 16 ? 16 : (ch > kMaxChunk ? kMaxChunk : ch);
+  int64_t cap = 2048 / batch;
+  cap = cap < 8 ? 8 : (cap > 128 ? 128 : cap);
+  int64_t ns = ceil_div(pages, ch);
+  *nsplit = (int)(ns < 2 ? 2 : (ns > cap ? cap : ns));
+  *chunk = (int)ch;
+}
+
+size_t decode_rows_workspace_bytes(int batch, int hq, int hkv, int64_t pages) {
+  int ns, ch;
+  decode_rows_plan(batch, hkv, pages, &ns, &ch);
+  return decode_workspace_bytes(batch, hq, ns, true);
+}
+
+namespace {
+template <int DT, int G>
+void launch_rows_g(const DecodeArgs &a, int units, hipStream_t stream) {
+  const size_t sm = (size_t)kHeadMajorWaves * (kVTile * sizeof(uint16_t) + G * (2 + kHeadDim) * sizeof(float));
+  hipLaunchKernelGGL((paged_decode_rows_kernel<DT, G>), dim3(units, a.hkv), dim3(64 * kHeadMajorWaves), sm, stream, a);
+}
+template <int DT>
+void launch_decode_rows(const DecodeArgs &a, int G, int units, hipStream_t stream) {
+  switch (G) {
+    case 1: launch_rows_g<DT, 1>(a, units, stream); break;
+    case 2: launch_rows_g<DT, 2>(a, units, stream); break;
+    case 3: launch_rows_g<DT, 3>(a, units, stream); break;
+    case 4: launch_rows_g<DT, 4>(a, units, stream); break;
+    case 5: launch_rows_g<DT, 5>(a, units, stream); break;
+    case 6: launch_rows_g<DT, 6>(a, units, stream); break;
+    case 7: launch_rows_g<DT, 7>(a, units, stream); break;
+    default: launch_rows_g<DT, 8>(a, units, stream); break;
+  }
+  hipLaunchKernelGGL((decode_merge_kernel<DT, true>), dim3(a.batch * a.hq), dim3(kHeadDim * merge_groups(a.nsplit)), 0,
+                     stream, a, G);
+}
+}  // namespace
+
+// Arguments as delta_paged_prefill, checked there; workspace of decode_rows_workspace_bytes, 256-byte aligned.
+int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache, int64_t num_pages,
+                    const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices,
+                    int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o, int64_t o_stride_t,
+                    int64_t o_stride_h, float *lse, int batch, int hq, int hkv, int dtype, float sm_scale,
+                    void *workspace, hipStream_t stream, const char *who) {
+  DecodeArgs a = {};
+  a.q = (const uint16_t *)q;
+  a.q_stride_b = q_stride_t;
+  a.q_stride_h = q_stride_h;
+  a.kv = (const uint16_t *)kv_cache;
+  a.num_pages = num_pages;
+  a.kv_indptr = kv_indptr;
+  a.kv_indices = kv_indices;
+  a.kv_indices_len = kv_indices_len;
+  a.last_page_len = kv_last_page_len;
+  a.q_rows = qo_indptr;
+  a.o = (uint16_t *)o;
+  a.o_stride_b = o_stride_t;
+  a.o_stride_h = o_stride_h;
+  a.lse = lse;
+  a.batch = batch;
+  a.hq = hq;
+  a.hkv = hkv;
+  a.hb = 1;
+  a.sm_scale = sm_scale;
+  decode_rows_plan(batch, hkv, kv_indices_len, &a.nsplit, &a.chunk);
+  a.part_ml = (float *)workspace;
+  a.part_acc = a.part_ml + (size_t)batch * hq * a.nsplit * 2;
+  // Every row's units: its full ones (kv_indices_len / chunk in all) and its last one.
+  const int units = (int)(kv_indices_len / a.chunk) + batch;
+  if (dtype == DELTA_BF16)
+    launch_decode_rows<DELTA_BF16>(a, hq / hkv, units, stream);
+  else
+    launch_decode_rows<DELTA_FP16>(a, hq / hkv, units, stream);
   return check_launch(who);
 }
 

@@ -5,16 +5,30 @@
 // cache already holds the row's new tokens (update_kv runs before attention, model.py:413-418),
 // so query i of row b sits at position kv_len_b - qo_len_b + i and attends tokens 0..position.
 //
-// Work decomposition (flash-attention style, on 32x32 MFMA tiles): a block is kPW waves of one
+// Work decomposition (flash-attention style, on 32x32 MFMA tiles): a block is PW waves of one
 // (row, kv head) and a run of consecutive query tokens; each wave owns 32 query rows, the
 // (token, q head) pairs of TW = 32 / G tokens (rows past TW * G idle when G does not divide
 // 32), with its q in registers.  The block sweeps the row's kv tokens 64 at a time (four pages,
 // two 32-token sub-tiles) up to its last token's position: each step's K and V (16 KiB each for
-// one head) are loaded once per block, 16 bytes per thread, into padded LDS tiles (three
-// buffers; the next step in flight in registers) and read by every wave.  Waves 0-3 run each
-// step whole; waves 4-7, the second wave of each SIMD, run half a step behind (P.V of the
-// previous step, then S and softmax of this one, the previous step's V still in its buffer), so
-// the two waves of a SIMD are not both in their softmax at once.  Per wave and sub-tile:
+// one head) go from global memory straight to LDS (global_load_lds: no registers, no LDS store
+// instructions) and are read by every wave.
+//   PW = 8 (prompts of 4096 tokens and more): one block per CU, four step buffers.  Waves 0-3 run each
+//     step whole; waves 4-7, the second wave of each SIMD, run half a step behind (P.V of the
+//     previous step, then S and softmax of this one), so the two waves of a SIMD are not both in
+//     their softmax at once.  Steps are loaded two ahead.
+//   PW = 4: two blocks per CU, two step buffers each, the next step's loads issued under this step's
+//     MFMAs.  Half the tile: less idle time at the ends of short prompts, and one block's start runs
+//     under the other's steps.
+// What bounds it: MFMA and VALU issue of two waves per SIMD that overlap in part (without the MFMAs an
+// 8192-token prompt takes 390-410 us of 500-520, without the exponentials 475, without the loads 500),
+// under a clock that MFMA-heavy kernels pull down (a 16384^3 bf16 product reaches 1.57 PFLOP/s on this
+// card; this kernel 1.06).  Llama-3-8B shape, graph-free launches, us (registers-staged 8-wave kernel
+// before / PW 8 / PW 4): 8192 tokens 545 / 500 / 534, 2048 tokens 66 / 59 / 55, 300 tokens - / 15.5 /
+// 13.1, 8 prompts of 128-1024 - / 54 / 52.6, 32 prompts of 64-256 - / 42 / 35.  Of that, the fences
+// that keep fragment reads ahead of their MFMAs took 595 -> 571 (8192 tokens, with RoPE + append), the
+// scalar work of the loads (one check for invalid pages per block instead of one per step) 2048 tokens
+// 63 -> 58.  Prefetching a step's first K and V fragments in the step before: no gain (522 vs 516).
+// Per wave and sub-tile:
 //   S^T = K Q^T : 8 v_mfma_f32_32x32x16 over d, A = the tile's K rows from LDS
 //         (lane%32 = kv token, d in 16 ks + 8 (lane / 32) + [0, 8)), B = the wave's q (same d
 //         split, n = lane%32 = query row); D leaves lane l with its row n = l%32 and the 16 kv
@@ -29,26 +43,33 @@
 //         packed by v_cvt_pk_bf16_f32 / v_cvt_pk_f16_f32, A = V^T read from the padded tile
 //         with ds_read_b64_tr_b16 in that same kv order; lane l accumulates
 //         O[row l%32][d = 32 dt + 8 (i / 4) + 4 (l / 32) + i % 4].
-// LDS row pitches: K rows are read 16 bytes per lane, 32 rows at once (136 elements = 68 banks
-// apart: each 16-lane group covers the 64 banks once); V is read transposed, 4 rows x 16
-// columns per 16-lane group and two groups per pass (160 elements: consecutive rows 16 banks
-// apart, so a pass covers 64 banks once; at 136 consecutive rows share 4 banks: 2-way conflicts).
-// Blocks run heaviest first (the last query tiles attend the most tokens) and blockIdx.x is the
-// kv head, so the blocks of one head land on the same XCD (blocks go to the XCDs round robin)
-// and share its L2 for that head's K/V.  Page ids are preloaded 64 per register, with a bit
-// mask of the invalid ones.  No merge.
+// LDS tiles: 64 rows of 256 bytes, 16-byte chunks swizzled by row so that the fragment reads cover
+// the banks once (see the step loads).  Page ids come by scalar loads, a step ahead.
+// Blocks run heaviest first (the last query tiles attend the most tokens), the kv head fastest, so
+// with 8 kv heads the blocks of one head land on the same XCD (blocks go to the XCDs round robin)
+// and share its L2 for that head's K/V.  Up to 6144 kv tokens all rows run together, past that in groups
+// of about 3072: one row at a time leaves the last rows' heavy tiles to the end (8 prompts of 37-1500,
+// 5.5 k tokens: 71.4 vs 64.5 us), too many rows at once overflow the L2 (16 prompts of 512: all 93.3 us,
+// 8 rows 73.8, 4 rows 65.9, one 69.4).  No merge.
 #include "delta_common.h"
 
 namespace delta {
+
+int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache, int64_t num_pages,
+                    const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices,
+                    int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o, int64_t o_stride_t,
+                    int64_t o_stride_h, float *lse, int batch, int hq, int hkv, int dtype, float sm_scale,
+                    void *workspace, hipStream_t stream, const char *who);
+size_t decode_rows_workspace_bytes(int batch, int hq, int hkv, int64_t pages);
+
 namespace {
 
-constexpr int kPW = 8;          // waves per block (each 32 query rows)
 constexpr int kSub = 2;         // 32-token sub-tiles per step
 constexpr int kKvStep = 32 * kSub;  // kv tokens per step
 constexpr int kPgStep = kKvStep / 16;  // pages per step
-constexpr int kRowP = 136;      // padded K tile row (elements): conflict-free 16-byte row reads
-constexpr int kRowPV = 160;     // padded V tile row (elements), read transposed
-constexpr int kBufs = 3;        // LDS step buffers (late waves read a step after the next barrier)
+constexpr int kWideQo = 4096;   // longest prompt from which blocks hold 8 waves
+constexpr int kGroupTokens = 3072;  // kv tokens of the rows whose blocks run together (see the block order)
+constexpr int kTileB = kKvStep * 256;  // bytes of a step's K (or V) tile: 64 rows of 256 bytes
 
 struct PrefillArgs {
   const uint16_t *q;
@@ -64,6 +85,7 @@ struct PrefillArgs {
   int64_t o_stride_t, o_stride_h;
   float *lse;
   int batch, hq, hkv;
+  int skip_single;  // rows of one query token are run_decode_rows'
   float sm_scale;
 };
 
@@ -114,25 +136,32 @@ __device__ __forceinline__ float halves_sum(float v) {
   return __uint_as_float(x[0]) + __uint_as_float(x[1]);
 }
 
-template <int DT, int G>
-__global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) {
+template <int DT, int G, int PW>
+__global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a) {
 #pragma clang fp contract(off)
   using MF = Mfma32<DT>;
   constexpr int TW = 32 / G;                  // query tokens per wave
-  constexpr int BT = kPW * TW;                // query tokens per block
-  constexpr int kTile = kKvStep * kRowP;      // the K tile (elements); the V tile follows
-  constexpr int kTileV = kKvStep * kRowPV;
-  // Two step buffers, each K then V (padded rows), shared by the block's waves.
-  __shared__ uint16_t tiles[kBufs][kTile + kTileV];
+  constexpr int BT = PW * TW;                 // query tokens per block
+  constexpr bool kLate = PW == 8;             // the second wave of each SIMD runs half a step behind
+  // LDS step buffers: this step and the next, in flight; kLate also the late waves' step and one more
+  // in flight.
+  constexpr int kBufs = kLate ? 4 : 2;
+  constexpr int kPgWave = 16 / PW;            // pages a wave loads rows of, per step
+  // Step buffers, each the K tile, then the V tile (swizzled rows), shared by the block's waves.
+  __shared__ __attribute__((aligned(1024))) char tiles[kBufs][2 * kTileB];
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int hl = lane >> 5, n = lane & 31;
-  const int h = blockIdx.x, b = blockIdx.z;
+  // Blocks run in groups of gridDim.x / hkv rows (blockIdx.z).  Within a group the rows rotate by tile: blocks go to the XCDs round robin, and with fewer
+  // than 8 kv heads a fixed order would give an XCD all tiles of the same rows.
+  const int h = (int)blockIdx.x % a.hkv, grp_rows = (int)gridDim.x / a.hkv;
+  const int b = (int)blockIdx.z * grp_rows + (int)((blockIdx.x / a.hkv + blockIdx.y) % grp_rows);
+  if (b >= a.batch) return;
   const int64_t q0 = a.qo_indptr[b], q1 = a.qo_indptr[b + 1];
   const int qn = q1 > q0 ? (int)(q1 - q0) : 0;
-  const int tile = (int)gridDim.y - 1 - (int)blockIdx.y;  // heaviest tiles first
+  const int tile = (int)gridDim.y - 1 - (int)blockIdx.y;
   const int btok0 = tile * BT;
-  if (btok0 >= qn) return;  // whole block
+  if (btok0 >= qn || (a.skip_single && qn == 1)) return;  // whole block
   // The wave's first query token, read as a scalar: the compiler cannot see that wave (from the
   // thread index) is uniform, and with tok0 scalar the wave's step count and its diagonal test
   // (full / masked step) become scalar branches (8192-token prompt 594 -> 569-585 us).
@@ -177,74 +206,65 @@ __global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) 
   // First query position of the wave: steps ending at or below it need no causal mask.
   const int wpos0 = kv_len - qn + tok0;
 
-  const int64_t row_elems = (int64_t)a.hkv * kHeadDim;
-  const int64_t page_bytes = 2 * kPageSize * row_elems * 2;
-  // Cooperative step load: 2 * kKvStep * 16 chunks of 16 bytes (K, then V; rows x 16 chunks) over
-  // kPW * 64 threads.  Thread t stages chunk c16 = t % 16 of step rows t / 16 and t / 16 + 32 of
-  // K and of V; the 64 lanes of a wave cover four rows of one page, so the page of each of its
-  // loads is wave-uniform (page wave / 4 of the step for rows < 32, wave / 4 + 2 above): its id
-  // and base address are scalars and the lanes' offsets are fixed for the whole sweep.
-  constexpr int kChunks = 2 * kKvStep * (kHeadDim / 8);
-  constexpr int kPer = kChunks / (kPW * 64);
-  static_assert(kPer == 4 && kKvStep == 64 && kPW * 64 == 2 * kKvStep * 4, "staging layout");
-  const int wq = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 8));  // wave / 4
-  const int srow = (int)(threadIdx.x >> 4), c16 = (int)(threadIdx.x & 15);  // srow in [0, 32)
-  const uint32_t goff_k = (uint32_t)(((srow & 15) * row_elems + (int64_t)h * kHeadDim + 8 * c16) * 2);
-  const uint32_t goff_v = goff_k + (uint32_t)(kPageSize * row_elems * 2);
-  int lds_off[kPer];  // elements: K rows srow, srow + 32, then the padded V rows
+  // Step loads: K and V rows go straight to LDS, 1 KiB (4 rows of this head) per load, four loads
+  // per wave: K rows 4 wave .. + 3 and 32 above, then the same V rows.  The rows of a load lie in
+  // one page, so its base address is scalar and the lanes' offsets are fixed for the whole sweep.
+  // 16-byte chunk ch of K row r sits at slot ch ^ (r % 16) and of V row r at ch ^ 4 (r % 4): the
+  // K fragment reads (32 rows, one chunk) and the transposed V reads (4 rows x 64 bytes per 32
+  // lanes) then cover the banks once.
+  const uint32_t row_bytes = (uint32_t)a.hkv * kHeadDim * 2;
+  const uint32_t page_bytes = 2 * kPageSize * row_bytes;
+  const int wv = uniform((int)(threadIdx.x >> 6));
+  const int lrow = lane >> 4, lch = lane & 15;
+  const uint32_t koff = (4 * (wv & 3) + lrow) * row_bytes + 16 * (lch ^ (4 * (wv & 3) + lrow));
+  const uint32_t voff = (kPageSize + 4 * (wv & 3) + lrow) * row_bytes + 16 * (lch ^ (4 * lrow));
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char *)&tiles[0][0] + wv * 1024;
+  const char *const kvh = reinterpret_cast<const char *>(a.kv) + (int64_t)h * (kHeadDim * 2);
+  // Page ids outside the cache (negative or past it) are looked for once, over all pages the block
+  // sweeps: the steps of a row without any (the usual case) take its ids as they are.
+  const int32_t *const row_ids = a.kv_indices + p0;
+  auto page_bad = [&](int pid) { return pid < 0 || (int64_t)pid >= a.num_pages; };
+  bool row_bad = false;
+  for (int i = 0; i < nsteps * kPgStep && i < np; i += 64)
+    row_bad |= __ballot(i + lane < np && page_bad(row_ids[i + lane < np ? i + lane : 0])) != 0;
+  auto bad_of = [&](int j) {  // bit i: page i of step j lies outside the cache
+    uint32_t r = 0;
 #pragma unroll
-  for (int r = 0; r < kPer; ++r)
-    lds_off[r] = (r < 2 ? (srow + 32 * r) * kRowP : kTile + (srow + 32 * (r - 2)) * kRowPV) + 8 * c16;
-
-  // Page ids, 64 per register (lane i: page cbase + i), the next 64 a chunk ahead.
-  const int npages = (nsteps * kKvStep + kPageSize - 1) / kPageSize;
-  auto load_ids = [&](int base) -> int {
-    const int it = base + lane;
-    int pid = -1;
-    if (it < npages && it < np) pid = a.kv_indices[p0 + it];
-    return (pid >= 0 && (int64_t)pid < a.num_pages) ? pid : -1;
+    for (int i = 0; i < kPgStep; ++i) {
+      const int pg = kPgStep * j + i;
+      r |= (pg < np && page_bad(ld_scalar(row_ids, pg < np ? pg : np - 1)) ? 1u : 0u) << i;
+    }
+    return r;
   };
-  // Invalid page ids (negative or past the cache) of the current window, one bit per page.
-  const int lim = npages < np ? npages : np;
-  auto bad_of = [&](int id, int base) -> uint64_t { return __ballot(base + lane < lim && id < 0); };
-  int cbase = 0;
-  int ids = npages > 0 ? load_ids(0) : -1;
-  int ids_next = npages > 64 ? load_ids(64) : -1;
-  uint64_t bad = bad_of(ids, 0);
-  auto id_of = [&](int pg) -> int {  // pg in [cbase, cbase + 128)
-    return pg - cbase < 64 ? __builtin_amdgcn_readlane(ids, pg - cbase) : __builtin_amdgcn_readlane(ids_next, pg - cbase - 64);
-  };
-  u32x4 ring[kPer];  // K rows srow, srow + 32, V rows srow, srow + 32
-  auto fetch = [&](int j) {  // global loads of step j into the ring
+  // The pages the wave loads four rows of in step j: page (wave / 4) + i PW / 4 of its four; pages
+  // past the row repeat its last one (masked later).
+  const uint32_t last_pg = (uint32_t)(np - 1);
+  uint32_t id[kPgWave];  // of the step issued next
+  auto load_ids = [&](int j) {
 #pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const int pg = kPgStep * j + wq + 2 * half;
-      const int pid = pg < npages ? id_of(pg) : -1;
-      if (pid >= 0) {
-        const char *pb = reinterpret_cast<const char *>(a.kv) + (int64_t)pid * page_bytes;
-        ring[half] = ld128(pb + goff_k);
-        ring[2 + half] = ld128(pb + goff_v);
-      } else {
-        ring[half] = u32x4{0u, 0u, 0u, 0u};
-        ring[2 + half] = u32x4{0u, 0u, 0u, 0u};
-      }
+    for (int i = 0; i < kPgWave; ++i) {
+      const uint32_t pg = (uint32_t)(kPgStep * j + i * (PW / 4) + (wv >> 2));
+      id[i] = (uint32_t)ld_scalar(row_ids, pg < last_pg ? pg : last_pg);
     }
   };
-  auto stage = [&](int j) {  // the ring (step j) into tiles[j % kBufs]; V rows past kv_len as zeros
-    uint16_t *tb = &tiles[j % kBufs][0];
-    const bool v_whole = (j + 1) * kKvStep <= kv_len;
+  auto issue = [&](int j, int i) {
+    const uint32_t dst = lds0 + (uint32_t)(j % kBufs) * (2 * kTileB) + i * (PW / 4) * 4096;
+    const uint32_t pid = row_bad && page_bad((int)id[i]) ? 0u : id[i];
+    const char *pg = kvh + (uint64_t)pid * page_bytes;
+    load_lds_1k(dst, pg, koff);
+    load_lds_1k(dst + kTileB, pg, voff);
+  };
+  auto issue_step = [&](int j) {  // step j's loads, then the ids of step j + 1
 #pragma unroll
-    for (int r = 0; r < kPer; ++r) {
-      u32x4 v = ring[r];
-      if (r >= 2 && !v_whole && j * kKvStep + srow + 32 * (r - 2) >= kv_len) v = u32x4{0u, 0u, 0u, 0u};
-      st128(tb + lds_off[r], v);
-    }
+    for (int i = 0; i < kPgWave; ++i) issue(j, i);
+    load_ids(j + 1);
   };
   if (nsteps > 0) {
-    fetch(0);
-    stage(0);
-    if (nsteps > 1) fetch(1);
+    load_ids(0);
+    issue_step(0);
+    if (kLate && nsteps > 1) issue_step(1);
   }
+  uint32_t bad = 0;  // bad_of(j)
 
   float m = -INFINITY, l = 0.f;
   f32x16 acc[4];
@@ -253,45 +273,55 @@ __global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) 
 #pragma unroll
     for (int i = 0; i < 16; ++i) acc[dt][i] = 0.f;
   const float scale2 = fabsf(a.sm_scale) * kLog2e;
+  // K fragment of k-slice ks: row 32 sb + n, chunk 2 ks + hl.
+  uint32_t kfo[8];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) kfo[ks] = (uint32_t)(n * 256 + 16 * ((2 * ks + hl) ^ (n & 15)));
   // ds_read_b64_tr_b16 of V^T: 16-lane group q16 = lane / 16, t16 = lane % 16 reads rows
-  // (kv) base + t16 / 4 at columns 16 (q16 % 2) + 4 (t16 % 4), and receives its column's four rows.
+  // (kv) base + t16 / 4 at columns 32 dt + 16 (q16 % 2) + 4 (t16 % 4), and receives its column's four rows.
   const int q16 = lane >> 4, t16 = lane & 15;
-  const int vtr_off = kTile + (4 * hl + (t16 >> 2)) * kRowPV + 16 * (q16 & 1) + 4 * (t16 & 3);
+  uint32_t vfo[4];
+#pragma unroll
+  for (int dt = 0; dt < 4; ++dt)
+    vfo[dt] = (uint32_t)(kTileB + (4 * hl + (t16 >> 2)) * 256 +
+                         16 * ((4 * dt + 2 * (q16 & 1) + ((t16 & 3) >> 1)) ^ (4 * (t16 >> 2))) + 8 * (t16 & 1));
 
   // One step for the wave: S^T = K Q^T, the online softmax (accumulators rescaled when the
   // reference maximum moves) and P^T packed into pc.
-  auto score_step = [&](int j, const uint16_t *tk, u32x4 (&pc)[2 * kSub]) {
+  auto score_step = [&](int j, const char *tk, u32x4 (&pc)[2 * kSub]) {
     f32x16 S[kSub];
 #pragma unroll
     for (int sb = 0; sb < kSub; ++sb)
 #pragma unroll
       for (int i = 0; i < 16; ++i) S[sb][i] = 0.f;
-    // K fragments two k-slices ahead of the MFMAs that use them (one ahead: 2048 tokens ~1 %
-    // slower, same registers).
-    auto kfrag = [&](int sb, int ks) { return *reinterpret_cast<const u32x4 *>(tk + (32 * sb + n) * kRowP + 16 * ks + 8 * hl); };
-    u32x4 kq[3][kSub];  // fragments of k-slices ks, ks + 1, ks + 2
+    // K fragments three k-slices ahead of the MFMAs that use them; the fences keep the compiler from
+    // sinking each read to its use, where every slice would wait out the LDS latency.
+    auto kfrag = [&](int sb, int ks) { return *reinterpret_cast<const u32x4 *>(tk + kfo[ks] + sb * 8192); };
+    u32x4 kq[4][kSub];
 #pragma unroll
-    for (int s = 0; s < 2; ++s)
+    for (int s = 0; s < 3; ++s)
 #pragma unroll
       for (int sb = 0; sb < kSub; ++sb) kq[s][sb] = kfrag(sb, s);
+    __builtin_amdgcn_sched_barrier(0);
     // Raised wave priority over each MFMA run: of the SIMD's two waves, the one with MFMAs
-    // to issue goes first, which pushes the other into its softmax meanwhile (~1 %).
+    // to issue goes first, which pushes the other into its softmax meanwhile (8192 tokens 569 -> 517 us).
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
-      if (ks + 2 < 8) {
+      if (ks + 3 < 8) {
 #pragma unroll
-        for (int sb = 0; sb < kSub; ++sb) kq[(ks + 2) % 3][sb] = kfrag(sb, ks + 2);
+        for (int sb = 0; sb < kSub; ++sb) kq[(ks + 3) % 4][sb] = kfrag(sb, ks + 3);
       }
 #pragma unroll
-      for (int sb = 0; sb < kSub; ++sb) S[sb] = MF::run(kq[ks % 3][sb], qf[ks], S[sb]);
+      for (int sb = 0; sb < kSub; ++sb) S[sb] = MF::run(kq[ks % 4][sb], qf[ks], S[sb]);
+      if (!kLate && ks < kPgWave && j + 1 < nsteps) issue(j + 1, ks);  // the next step's loads go out under the MFMAs
+      __builtin_amdgcn_sched_barrier(0);
     }
+    if (!kLate && j + 1 < nsteps) load_ids(j + 2);
     __builtin_amdgcn_s_setprio(0);
     // Masks only where the step crosses the wave's first diagonal, kv_len, or a bad page.
     const int kv0 = j * kKvStep;
-    const int poff = kPgStep * j - cbase;  // the step's pages: bits poff .. poff + kPgStep - 1
-    const bool pages_ok = ((bad >> poff) & ((1ull << kPgStep) - 1)) == 0;
-    const bool full = kv0 + kKvStep - 1 <= wpos0 && kv0 + kKvStep <= kv_len && pages_ok;
+    const bool full = kv0 + kKvStep - 1 <= wpos0 && kv0 + kKvStep <= kv_len && bad == 0;
     // Row maxima on the raw scores (the scale is positive, so it commutes with max), then
     // x = S * scale - m as one fma.  m is the row's reference maximum: it moves only when a
     // score exceeds it by more than 8 (a factor of 2^8), so the exponentials stay <= 256 and the
@@ -308,7 +338,7 @@ __global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) 
     } else {
       bool pg_ok[kPgStep];
 #pragma unroll
-      for (int p = 0; p < kPgStep; ++p) pg_ok[p] = ((bad >> (poff + p)) & 1ull) == 0;
+      for (int p = 0; p < kPgStep; ++p) pg_ok[p] = ((bad >> p) & 1u) == 0;
 #pragma unroll
       for (int i = 0; i < NX; ++i) {
         const int mm = 32 * (i >> 4) + 8 * ((i & 15) >> 2) + 4 * hl + (i & 3);
@@ -345,41 +375,63 @@ __global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) 
         pc[cc][w] = pack2<DT>(x[8 * cc + 2 * w], x[8 * cc + 2 * w + 1]);
   };
   // O^T += V^T P^T of a step whose P^T is in pc.
-  auto pv_step = [&](const uint16_t *tk, const u32x4 (&pc)[2 * kSub]) {
+  auto pv_step = [&](const char *tk, const u32x4 (&pc)[2 * kSub]) {
+    auto vfrag = [&](int i) {  // V^T fragment of chunk i / 4, d tile i % 4
+      const char *rd = tk + vfo[i % 4] + (i / 4) * 4096;
+      const ps4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ps4_t *)rd);
+      const ps4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ps4_t *)(rd + 2048));
+      u32x4 va;
+      va[0] = (uint32_t)(uint16_t)v0[0] | ((uint32_t)(uint16_t)v0[1] << 16);
+      va[1] = (uint32_t)(uint16_t)v0[2] | ((uint32_t)(uint16_t)v0[3] << 16);
+      va[2] = (uint32_t)(uint16_t)v1[0] | ((uint32_t)(uint16_t)v1[1] << 16);
+      va[3] = (uint32_t)(uint16_t)v1[2] | ((uint32_t)(uint16_t)v1[3] << 16);
+      return va;
+    };
+    constexpr int kAhead = 4;  // fragments read ahead of their MFMAs
+    u32x4 vq[kAhead + 1];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) vq[i] = vfrag(i);
+    __builtin_amdgcn_sched_barrier(0);
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
-    for (int dt = 0; dt < 4; ++dt)
-#pragma unroll
-      for (int cc = 0; cc < 2 * kSub; ++cc) {
-        const uint16_t *rd = tk + vtr_off + 16 * cc * kRowPV + 32 * dt;
-        const ps4_t v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ps4_t *)rd);
-        const ps4_t v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_ps4_t *)(rd + 8 * kRowPV));
-        u32x4 va;
-        va[0] = (uint32_t)(uint16_t)v0[0] | ((uint32_t)(uint16_t)v0[1] << 16);
-        va[1] = (uint32_t)(uint16_t)v0[2] | ((uint32_t)(uint16_t)v0[3] << 16);
-        va[2] = (uint32_t)(uint16_t)v1[0] | ((uint32_t)(uint16_t)v1[1] << 16);
-        va[3] = (uint32_t)(uint16_t)v1[2] | ((uint32_t)(uint16_t)v1[3] << 16);
-        acc[dt] = MF::run(va, pc[cc], acc[dt]);
-      }
+    for (int i = 0; i < 8 * kSub; ++i) {
+      if (i + kAhead < 8 * kSub) vq[(i + kAhead) % (kAhead + 1)] = vfrag(i + kAhead);
+      acc[i % 4] = MF::run(vq[i % (kAhead + 1)], pc[i / 4], acc[i % 4]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
     __builtin_amdgcn_s_setprio(0);
   };
 
-  // Waves 0-3 (one per SIMD) run each step whole; waves 4-7, the SIMDs' second waves, run half
+  // (PW = 8) Waves 0-3 (one per SIMD) run each step whole; waves 4-7, the SIMDs' second waves, run half
   // a step behind: P.V of the previous step first, then S and the softmax of this one.  So on
   // each SIMD one wave's softmax runs while the other wave's MFMAs do (P.V of one under the
   // other's softmax, S of one under the other's softmax), not both softmaxes at once.  A step's
-  // tiles stay in LDS for one more step (three buffers): the late waves read step j - 1 after
-  // the barrier of step j.
-  const bool late = wave >= kPW / 2;
+  // tiles stay in LDS for one more step: the late waves read step j - 1 after the barrier of step j.
+  const bool late = kLate && wave >= PW / 2;
   u32x4 pcar[2 * kSub];
-  for (int j = 0; j <= nsteps; ++j) {
-    __syncthreads();  // step j is in tiles[j % 3]; tiles[(j + 1) % 3] is free
-    if (j < nsteps && kPgStep * j >= cbase + 64) {  // the id window moves on
-      cbase += 64;
-      ids = ids_next;
-      bad = bad_of(ids, cbase);
-      ids_next = cbase + 64 < npages ? load_ids(cbase + 64) : -1;
+  for (int j = 0; nsteps > 0 && j < nsteps + (kLate ? 1 : 0); ++j) {
+    // Step j's loads have landed when at most the next step's (kLate: four) are pending.
+    if (kLate && j + 1 < nsteps)
+      wait_loads<2 * kPgWave>();
+    else
+      wait_loads<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (row_bad) bad = j < nsteps ? bad_of(j) : 0u;
+    if (j < nsteps && ((j + 1) * kKvStep > kv_len || bad != 0)) {
+      // V rows past kv_len and of pages outside the cache meet p = 0 but may hold NaN/Inf: zeros.
+      constexpr int kTpr = PW;  // threads per row
+      const int r = (int)threadIdx.x / kTpr;
+      if (j * kKvStep + r >= kv_len || ((bad >> (r >> 4)) & 1u)) {
+        char *vr = &tiles[j % kBufs][kTileB + r * 256 + 256 / kTpr * ((int)threadIdx.x % kTpr)];
+#pragma unroll
+        for (int i = 0; i < 16 / kTpr; ++i) st128(vr + 16 * i, u32x4{0u, 0u, 0u, 0u});
+      }
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
     }
+    if (kLate ? j + 2 < nsteps : j >= wsteps && j + 1 < nsteps) issue_step(kLate ? j + 2 : j + 1);
     if (late) {
       if (j >= 1 && j - 1 < wsteps) pv_step(&tiles[(j - 1) % kBufs][0], pcar);
       if (j < wsteps) score_step(j, &tiles[j % kBufs][0], pcar);
@@ -387,10 +439,6 @@ __global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) 
       u32x4 pc[2 * kSub];
       score_step(j, &tiles[j % kBufs][0], pc);
       pv_step(&tiles[j % kBufs][0], pc);
-    }
-    if (j + 1 < nsteps) {
-      stage(j + 1);
-      if (j + 2 < nsteps) fetch(j + 2);
     }
   }
 
@@ -412,36 +460,46 @@ __global__ void __launch_bounds__(kPW * 64) paged_prefill_kernel(PrefillArgs a) 
   }
 }
 
+template <int DT, int G>
+void launch_prefill_g(const PrefillArgs &a, int max_qo, hipStream_t stream) {
+  const bool wide = max_qo >= kWideQo;
+  const int bt = 32 / G * (wide ? 8 : 4);
+  const int64_t kv_tokens = a.kv_indices_len * kPageSize;
+  int64_t rows = kv_tokens <= 2 * kGroupTokens ? a.batch : kGroupTokens * (int64_t)a.batch / kv_tokens;
+  rows = rows < 1 ? 1 : (rows > a.batch ? a.batch : rows);
+  const dim3 grid((unsigned)(a.hkv * rows), (unsigned)ceil_div(max_qo, bt), (unsigned)ceil_div(a.batch, rows));
+  if (wide)
+    hipLaunchKernelGGL((paged_prefill_kernel<DT, G, 8>), grid, dim3(512), 0, stream, a);
+  else
+    hipLaunchKernelGGL((paged_prefill_kernel<DT, G, 4>), grid, dim3(256), 0, stream, a);
+}
+
 template <int DT>
 void launch_prefill(const PrefillArgs &a, int G, int max_qo, hipStream_t stream) {
-  const int tw = 32 / G;
-  const dim3 grid(a.hkv, (unsigned)ceil_div(max_qo, (int64_t)tw * kPW), a.batch);
-  const dim3 block(kPW * 64);
   switch (G) {
-    case 1: hipLaunchKernelGGL((paged_prefill_kernel<DT, 1>), grid, block, 0, stream, a); break;
-    case 2: hipLaunchKernelGGL((paged_prefill_kernel<DT, 2>), grid, block, 0, stream, a); break;
-    case 3: hipLaunchKernelGGL((paged_prefill_kernel<DT, 3>), grid, block, 0, stream, a); break;
-    case 4: hipLaunchKernelGGL((paged_prefill_kernel<DT, 4>), grid, block, 0, stream, a); break;
-    case 5: hipLaunchKernelGGL((paged_prefill_kernel<DT, 5>), grid, block, 0, stream, a); break;
-    case 6: hipLaunchKernelGGL((paged_prefill_kernel<DT, 6>), grid, block, 0, stream, a); break;
-    case 7: hipLaunchKernelGGL((paged_prefill_kernel<DT, 7>), grid, block, 0, stream, a); break;
-    default: hipLaunchKernelGGL((paged_prefill_kernel<DT, 8>), grid, block, 0, stream, a); break;
+    case 1: launch_prefill_g<DT, 1>(a, max_qo, stream); break;
+    case 2: launch_prefill_g<DT, 2>(a, max_qo, stream); break;
+    case 3: launch_prefill_g<DT, 3>(a, max_qo, stream); break;
+    case 4: launch_prefill_g<DT, 4>(a, max_qo, stream); break;
+    case 5: launch_prefill_g<DT, 5>(a, max_qo, stream); break;
+    case 6: launch_prefill_g<DT, 6>(a, max_qo, stream); break;
+    case 7: launch_prefill_g<DT, 7>(a, max_qo, stream); break;
+    default: launch_prefill_g<DT, 8>(a, max_qo, stream); break;
   }
 }
 
 }  // namespace
 }  // namespace delta
 
-extern "C" DELTA_EXPORT int delta_paged_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h,
-                                                const void *kv_cache, int64_t num_pages, const int32_t *qo_indptr,
-                                                const int32_t *kv_indptr, const int32_t *kv_indices,
-                                                int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o,
-                                                int64_t o_stride_t, int64_t o_stride_h, float *lse, int batch,
-                                                int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
-                                                float sm_scale, int max_qo_len, delta_stream_t stream) {
-  using namespace delta;
+namespace delta {
+namespace {
+// rows: rows of one query token go to run_decode_rows (workspace of decode_rows_workspace_bytes).
+int run_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache, int64_t num_pages,
+                const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices, int64_t kv_indices_len,
+                const int32_t *kv_last_page_len, void *o, int64_t o_stride_t, int64_t o_stride_h, float *lse, int batch,
+                int num_qo_heads, int num_kv_heads, int head_dim, int dtype, float sm_scale, int max_qo_len, bool rows,
+                void *workspace, size_t workspace_bytes, delta_stream_t stream, const char *who) {
   clear_error();
-  const char *who = "delta_paged_prefill";
   if (batch <= 0 || max_qo_len <= 0) return DELTA_OK;
   if (head_dim != kHeadDim) return set_error(DELTA_ERR_INVALID, "%s: head_dim must be 128", who);
   if (num_kv_heads <= 0 || num_qo_heads <= 0 || num_qo_heads % num_kv_heads)
@@ -475,9 +533,55 @@ extern "C" DELTA_EXPORT int delta_paged_prefill(const void *q, int64_t q_stride_
   a.hq = num_qo_heads;
   a.hkv = num_kv_heads;
   a.sm_scale = sm_scale;
+  a.skip_single = rows;
+  if (rows) {
+    const size_t need = decode_rows_workspace_bytes(batch, num_qo_heads, num_kv_heads, kv_indices_len);
+    if (!workspace || workspace_bytes < need)
+      return set_error(DELTA_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
+    if ((uintptr_t)workspace & 255u) return set_error(DELTA_ERR_INVALID, "%s: workspace must be 256-byte aligned", who);
+    const int rc = run_decode_rows(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
+                                   kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
+                                   num_kv_heads, dtype, sm_scale, workspace, (hipStream_t)stream, who);
+    if (rc || max_qo_len == 1) return rc;
+  }
   if (dtype == DELTA_BF16)
     launch_prefill<DELTA_BF16>(a, G, max_qo_len, (hipStream_t)stream);
   else
     launch_prefill<DELTA_FP16>(a, G, max_qo_len, (hipStream_t)stream);
   return check_launch(who);
+}
+}  // namespace
+}  // namespace delta
+
+extern "C" DELTA_EXPORT int delta_paged_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h,
+                                                const void *kv_cache, int64_t num_pages, const int32_t *qo_indptr,
+                                                const int32_t *kv_indptr, const int32_t *kv_indices,
+                                                int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o,
+                                                int64_t o_stride_t, int64_t o_stride_h, float *lse, int batch,
+                                                int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
+                                                float sm_scale, int max_qo_len, delta_stream_t stream) {
+  return delta::run_prefill(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
+                            kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
+                            num_kv_heads, head_dim, dtype, sm_scale, max_qo_len, false, nullptr, 0, stream,
+                            "delta_paged_prefill");
+}
+
+extern "C" DELTA_EXPORT size_t delta_paged_prefill_rows_workspace_bytes(int batch, int num_qo_heads, int num_kv_heads,
+                                                                        int64_t kv_indices_len) {
+  if (batch <= 0 || num_qo_heads <= 0 || num_kv_heads <= 0 || kv_indices_len < 0) return 0;
+  return delta::decode_rows_workspace_bytes(batch, num_qo_heads, num_kv_heads, kv_indices_len);
+}
+
+extern "C" DELTA_EXPORT int delta_paged_prefill_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h,
+                                                     const void *kv_cache, int64_t num_pages, const int32_t *qo_indptr,
+                                                     const int32_t *kv_indptr, const int32_t *kv_indices,
+                                                     int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o,
+                                                     int64_t o_stride_t, int64_t o_stride_h, float *lse, int batch,
+                                                     int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
+                                                     float sm_scale, int max_qo_len, void *workspace,
+                                                     size_t workspace_bytes, delta_stream_t stream) {
+  return delta::run_prefill(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
+                            kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
+                            num_kv_heads, head_dim, dtype, sm_scale, max_qo_len, true, workspace, workspace_bytes, stream,
+                            "delta_paged_prefill_rows");
 }

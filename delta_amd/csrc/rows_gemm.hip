@@ -37,21 +37,6 @@ struct RowsArgs {
   int inter;      // GLU: W = [gate rows; up rows], out [M][inter]
 };
 
-// 1 KiB from global memory straight into LDS: lane l's 16 bytes at base + off land at lds + 16 l.
-// Asynchronous (vmcnt); the compiler does not see the LDS write, the caller waits and fences.
-__device__ __forceinline__ void load_lds_1k(uint32_t lds, const void *base, uint32_t off, bool stream) {
-  if (stream)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(off), "s"(base)
-                 : "memory");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-                 : "memory");
-}
-template <int N>
-__device__ __forceinline__ void wait_loads() {  // at most N vector loads outstanding, LDS reads done
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(N) : "memory");
-}
-
 // A block: kg (2) x WM x WN waves; wave (kg, wm, wn) computes TM x TN tiles of 16 tokens x 16 W rows over
 // the k half kg of every 64-wide k step.
 template <int DT, int WM, int TM, int WN, int TN, int SK, int WS, bool GLU>
@@ -113,13 +98,13 @@ __global__ void __launch_bounds__(128 * WM * WN) gemm_rows_kernel(RowsArgs a) {
       const int q = wave + NW * j;
       int s = slab * SK + q / (kRows / 8);
       s = s < total ? s : total - 1;  // past the end: the last step again, never read
-      load_lds_1k(dst + q * 1024, xb + (int64_t)s * 128, xoff[j % XG], false);
+      load_lds_1k(dst + q * 1024, xb + (int64_t)s * 128, xoff[j % XG]);
     }
   };
   auto issue_w = [&](int s) {
     const uint32_t dst = lds_w + (uint32_t)(s % WS) * kWStage;
 #pragma unroll
-    for (int j = 0; j < LW; ++j) load_lds_1k(dst + (wave + NW * j) * 1024, wb + (int64_t)s * 128, woff[j], true);
+    for (int j = 0; j < LW; ++j) load_lds_1k<true>(dst + (wave + NW * j) * 1024, wb + (int64_t)s * 128, woff[j]);
   };
 
   f32x4 acc[TN][TM];

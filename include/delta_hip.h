@@ -213,6 +213,21 @@ int delta_paged_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h,
                         int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
                         float sm_scale, int max_qo_len, delta_stream_t stream);
 
+/* delta_paged_prefill for steps in which prompts join rows that are decoding: the same o and lse, with
+ * the rows of exactly one query token attended by split decode units (a merge launch follows) instead of
+ * one prefill block per kv head each.  workspace: delta_paged_prefill_rows_workspace_bytes bytes, 256-byte
+ * aligned. */
+size_t delta_paged_prefill_rows_workspace_bytes(int batch, int num_qo_heads, int num_kv_heads,
+                                                int64_t kv_indices_len);
+int delta_paged_prefill_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache,
+                             int64_t num_pages, const int32_t *qo_indptr, const int32_t *kv_indptr,
+                             const int32_t *kv_indices, int64_t kv_indices_len,
+                             const int32_t *kv_last_page_len, void *o, int64_t o_stride_t, int64_t o_stride_h,
+                             float *lse, int batch, int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
+                             float sm_scale, int max_qo_len, void *workspace, size_t workspace_bytes,
+                             delta_stream_t stream);
+
+
 /* ------------------------------------------------------------------------ */
 /* Page scoring (del3_legacy_softmax)                                         */
 /* ------------------------------------------------------------------------ */

@@ -1,0 +1,149 @@
+"""GPU: prompt steps with decoding rows (delta_paged_prefill_rows) against the plain prefill launch and
+fp64, and the block-order and page-check edges of the prefill kernel."""
+import random
+
+import pytest
+import torch
+
+from delta_amd import _lib, kernels as K
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def build(rows, hq, hkv, dtype, seed, spoil=True):
+    """rows: (new tokens, tokens after the step).  Slots past a row's end hold NaN when ``spoil``."""
+    rng = random.Random(seed)
+    counts = [n // 16 + 1 for _, n in rows]
+    perm = list(range(sum(counts) + 3))
+    rng.shuffle(perm)
+    gen = torch.Generator(device=DEV).manual_seed(seed)
+    kv = torch.randn((len(perm), 2, 16, hkv, 128), generator=gen, device=DEV).to(dtype)
+    ids, ptr, qo = [], [0], [0]
+    for (m, n), c in zip(rows, counts):
+        pages = perm[len(ids):len(ids) + c]
+        if spoil:
+            kv[pages[-1], :, n % 16:] = float("nan")
+        ids += pages
+        ptr.append(len(ids))
+        qo.append(qo[-1] + m)
+    i32 = dict(dtype=torch.int32, device=DEV)
+    q = torch.randn((max(qo[-1], 1), hq, 128), generator=gen, device=DEV).to(dtype)
+    return dict(q=q, kv=kv, qo=torch.tensor(qo, **i32), ptr=torch.tensor(ptr, **i32), ids=torch.tensor(ids, **i32),
+                last=torch.tensor([n % 16 for _, n in rows], **i32))
+
+
+def launch(c, rows, max_qo, scale=128 ** -0.5):
+    q, kv = c["q"], c["kv"]
+    hq, hkv, B = q.shape[1], kv.shape[3], c["qo"].numel() - 1
+    o = torch.full_like(q, 7.0)
+    lse = torch.full(q.shape[:2], 7.0, device=DEV)
+    args = [q.data_ptr(), q.stride(0), q.stride(1), kv.data_ptr(), kv.shape[0], c["qo"].data_ptr(), c["ptr"].data_ptr(),
+            c["ids"].data_ptr(), c["ids"].numel(), c["last"].data_ptr(), o.data_ptr(), o.stride(0), o.stride(1),
+            lse.data_ptr(), B, hq, hkv, 128, K._dtype_code(q), scale, max_qo]
+    stream = torch.cuda.current_stream().cuda_stream
+    if rows:
+        n = _lib.query("delta_paged_prefill_rows_workspace_bytes", B, hq, hkv, c["ids"].numel())
+        ws = torch.full((n,), 255, dtype=torch.uint8, device=DEV)  # NaN partials where none are written
+        _lib.call("delta_paged_prefill_rows", *args, ws.data_ptr(), n, stream)
+    else:
+        _lib.call("delta_paged_prefill", *args, stream)
+    torch.cuda.synchronize()
+    return o, lse
+
+
+CASES = {
+    "joins_g4": ([(77, 77)] + [(1, 1 + 97 * i) for i in range(20)], 32, 8, torch.bfloat16),
+    "joins_g7_chunked": ([(1, 3000), (40, 1040), (1, 1), (0, 64), (2, 50), (1, 16), (1, 17), (1, 2047)], 28, 4,
+                         torch.float16),
+    "one_row": ([(1, 5000)], 12, 2, torch.bfloat16),
+    "all_single_g1": ([(1, 10 + 300 * i) for i in range(9)], 4, 4, torch.float16),
+    "long_row_past_the_unit_cap_g8": ([(1, 40000)] + [(1, 33)] * 300 + [(5, 5)], 8, 1, torch.bfloat16),
+}
+
+
+@pytest.mark.parametrize("name", list(CASES))
+def test_prefill_rows_matches_prefill_and_fp64(name):
+    """Rows of other token counts keep the plain launch's bits; single-token rows agree within the two
+    kernels' roundings of P (2e-2, the attention tolerance) and with fp64 on sampled rows; lse to fp32."""
+    rows, hq, hkv, dtype = CASES[name]
+    c = build(rows, hq, hkv, dtype, seed=len(rows))
+    mx = max(m for m, _ in rows)
+    o0, l0 = launch(c, False, mx)
+    o1, l1 = launch(c, True, mx)
+    qo = c["qo"].tolist()
+    for b, (m, n) in enumerate(rows):
+        s = slice(qo[b], qo[b + 1])
+        if m != 1:
+            assert torch.equal(o0[s], o1[s]) and torch.equal(l0[s], l1[s])
+            continue
+        assert (o0[s].float() - o1[s].float()).abs().max().item() <= 2e-2
+        assert (l0[s] - l1[s]).abs().max().item() <= 1e-4
+    singles = [b for b, (m, _) in enumerate(rows) if m == 1]
+    for b in singles[:3] + singles[-2:]:
+        n = rows[b][1]
+        pages = c["ids"][c["ptr"][b]:c["ptr"][b + 1]].long()
+        kv = c["kv"][pages].double()
+        k, v = (kv[:, i].reshape(-1, hkv, 128)[:n] for i in (0, 1))
+        q = c["q"][qo[b]].double().view(hkv, hq // hkv, 128)
+        s = torch.einsum("hgd,nhd->hgn", q.cpu(), k.cpu()) * 128 ** -0.5
+        o = torch.einsum("hgn,nhd->hgd", s.softmax(-1), v.cpu()).reshape(hq, 128)
+        assert (o1[qo[b]].cpu().double() - o).abs().max().item() <= 2e-2
+
+
+def test_prefill_rows_zero_length_and_invalid_pages():
+    """A single-token row without pages gives zeros and -inf; ids outside the cache are masked, in the
+    prompt's steps and in the decoding rows, and their neighbours' NaN never reaches the output."""
+    rows = [(300, 300), (1, 700), (1, 200), (130, 900)]
+    c = build(rows, 32, 8, torch.bfloat16, seed=5)
+    ptr = c["ptr"].tolist()
+    for b, at in ((0, 3), (0, 18), (1, 40), (3, 0), (3, 30)):
+        c["ids"][ptr[b] + at] = -1 if at % 2 else c["kv"].shape[0]
+    c["kv"][0] = float("nan")  # page 0 stands in for an invalid id's address
+    used = (c["ids"] == 0).nonzero().flatten()
+    c["ids"][used] = c["kv"].shape[0] - 1
+    o0, l0 = launch(c, False, 300)
+    o1, l1 = launch(c, True, 300)
+    assert torch.isfinite(o0).all() and torch.isfinite(o1).all()
+    assert (o0.float() - o1.float()).abs().max().item() <= 2e-2 and (l0 - l1).abs().max().item() <= 1e-4
+    c["ptr"][3:] = c["ptr"][2].clone()  # rows 2 and 3: no pages
+    o1, l1 = launch(c, True, 300)
+    assert torch.all(o1[301] == 0) and torch.all(l1[301] == float("-inf"))
+
+
+@pytest.mark.parametrize("lens", [[5000, 4100], [64] * 40, [3, 700, 64, 65, 1, 2000, 511, 4095]])
+def test_prefill_block_orders_match_a_row_at_a_time(lens):
+    """8-wave blocks (4096 tokens and more), 4-wave blocks, rows in one group and in several: each row
+    equals the launch of that row alone, bit for bit where both use the same block size."""
+    c = build([(n, n) for n in lens], 28, 4, torch.bfloat16, seed=sum(lens))
+    o, lse = launch(c, False, max(lens))
+    qo, ptr = c["qo"].tolist(), c["ptr"].tolist()
+    for b, n in enumerate(lens):
+        one = dict(q=c["q"][qo[b]:qo[b + 1]].contiguous(), kv=c["kv"], qo=torch.tensor([0, n], dtype=torch.int32, device=DEV),
+                   ptr=torch.tensor([0, ptr[b + 1] - ptr[b]], dtype=torch.int32, device=DEV),
+                   ids=c["ids"][ptr[b]:ptr[b + 1]].contiguous(), last=c["last"][b:b + 1].contiguous())
+        o1, l1 = launch(one, False, max(lens) if max(lens) < 4096 else max(n, 4096))
+        assert torch.equal(o1, o[qo[b]:qo[b + 1]]) and torch.equal(l1, lse[qo[b]:qo[b + 1]])
+
+
+def test_paged_prefill_takes_the_rows_path_where_it_should():
+    assert K._prefill_has_decode_rows(808, 32, 777, 32 * 300)
+    assert K._prefill_has_decode_rows(4, 4, 1, 4 * 32)
+    assert not K._prefill_has_decode_rows(4, 4, 1, 4 * 32 - 1)     # short rows
+    assert not K._prefill_has_decode_rows(8192, 1, 8192, 513)      # one prompt
+    assert not K._prefill_has_decode_rows(8 * 1024, 8, 1024, 8 * 65)  # equal prompts
+    rows, hq, hkv, dtype = CASES["joins_g7_chunked"]
+    rows = [(m, n + 600 * (m > 0)) for m, n in rows]
+    c = build(rows, hq, hkv, dtype, seed=4)
+    args = (c["q"], c["kv"], c["qo"], c["ptr"], c["ids"], c["last"])
+    assert K._prefill_has_decode_rows(c["q"].shape[0], len(rows), 40, c["ids"].numel())
+    o = K.paged_prefill(*args, max_qo_len=40)
+    assert torch.equal(o, launch(c, True, 40)[0])
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        og = K.paged_prefill(*args, max_qo_len=40)
+    for _ in range(3):
+        og.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(og, o)
