@@ -1279,8 +1279,12 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
   }
   int64_t ch = max_pages > 0 ? ceil_div(max_pages, ns) : 1;
   if (ns > 1 && ch > kMaxChunk) {
+    // (Equal units instead of a short last one were slower for the dump launches: 64 rows of 517 pages,
+    // 2 kv heads, 256 blocks of 128 pages and 64 of 5: 104 us, 320 of 104: 116.)
     ch = kMaxChunk;
     ns = ceil_div(max_pages, ch);
+    // A dump launch's rest of a few pages goes to the unit before it instead of blocks of its own.
+    if (dump && ns > 1 && (max_pages - (ns - 1) * ch) * 16 <= kMaxChunk) --ns;
   }
   // Small launches whose units give each of 4 waves at most 8 pages (the config 2 and 4 subset
   // launches) run 4-wave blocks; when they split and 4x their split count still fits one 16-split
@@ -1288,9 +1292,7 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
   // (an unsplit launch keeps its blocks: no merge launch), each wave
   // storing its partial from registers with no closing block merge (config-2 subset 17.4 -> 16.6
   // us; at config 4, 16 -> 64 splits, the merge's 4x partials cost more than the block merge
-  // saves: 13.6 -> 14.2 us).  Others keep 16 waves (the config-4 full attention, 128-page units:
-  // with 4 waves its full-cache engine step ran 5.4-5.6 -> 5.9-6.0 ms, though a launch timed alone
-  // was unchanged).
+  // saves: 13.6 -> 14.2 us).
   if (small && ceil_div(ch, (int64_t)kHeadMajorWaves) <= 8) {
     R = kHeadMajorWaves;
     if (ns > 1 && ns * kHeadMajorWaves <= 16 && ns * kHeadMajorWaves <= max_pages) {
@@ -1298,6 +1300,18 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
       ch = ceil_div(max_pages, ns);
       R = 1;
     }
+  } else if (small && (int64_t)batch * hkv >= 32) {
+    // Longer units (full attention of small batches): about 1024 one-wave blocks, at least 4 waves per
+    // CU, each storing its partial from registers; a ragged batch's units stay short.  Against 16-wave
+    // blocks, with the merge: 64 rows of 513 pages, 2 kv heads (8 splits) 109.5 -> 87.0 us (in a decode
+    // step 106 -> 84.5 without it); 8 rows of 1025 pages, 8 kv heads 99.0 -> 87; 16 rows of 129 pages,
+    // 8 kv heads 30.3 -> 29.0.  Fewer than 32 (row, kv head) pairs would need more than 32 splits, whose
+    // partials the merge pays for, and keep 16-wave blocks: with 4 waves the config-4 full attention (4
+    // rows of 4097 pages, 4 kv heads) is as fast alone (90.5 vs 92.8 us) but slower in a step (103 vs 90).
+    ns = ceil_div(1024, (int64_t)batch * hkv);
+    if (ns < ceil_div(max_pages, kMaxChunk)) ns = ceil_div(max_pages, kMaxChunk);
+    ch = ceil_div(max_pages, ns);
+    R = 1;
   }
   *nsplit = (int)ns;
   *waves = h * R;
@@ -1499,15 +1513,16 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h, const void
 // The rows of exactly one query token of a prompt step (delta_paged_prefill_rows): decode attention of
 // those rows over packed head-major work units of 4-wave blocks, then the merge.  Row lengths are only
 // on the device; the host knows the pages of all rows together, so a unit holds what brings the launch to
-// about 1024 blocks, 16-128 pages (4-32 per wave), and a row has at most as many units as keep the
-// partials within 2048 (row, unit) slots (8 per row for more than 256 rows; a longer row's last unit
-// takes the rest).
+// about 1024 blocks, 16-128 pages (4-32 per wave), and a row has at most the units of four times the
+// average length (16 at least, 128 at most; a longer row's last unit takes the rest): the merge reads a
+// row's first 16 slots per group whether used or not (32 rows, 7 units each: 64 slots 10.5 us).
 void decode_rows_plan(int batch, int hkv, int64_t pages, int *nsplit, int *chunk) {
   int64_t ch = ceil_div(pages * hkv, 1024);
   ch = ch < 16 ? 16 : (ch > kMaxChunk ? kMaxChunk : ch);
-  int64_t cap = 2048 / batch;
-  cap = cap < 8 ? 8 : (cap > 128 ? 128 : cap);
+  int64_t cap = 128;
   int64_t ns = ceil_div(pages, ch);
+  const int64_t fit = 4 * ceil_div(ceil_div(pages, batch), ch);  // rows of four times the average length
+  cap = fit < 16 ? 16 : (fit < cap ? fit : cap);
   *nsplit = (int)(ns < 2 ? 2 : (ns > cap ? cap : ns));
   *chunk = (int)ch;
 }

@@ -126,6 +126,7 @@ def test_prefill_block_orders_match_a_row_at_a_time(lens):
         assert torch.equal(o1, o[qo[b]:qo[b + 1]]) and torch.equal(l1, lse[qo[b]:qo[b + 1]])
 
 
+@torch.inference_mode()  # as the engine captures: torch's graph state must not change mode between captures
 def test_paged_prefill_takes_the_rows_path_where_it_should():
     assert K._prefill_has_decode_rows(808, 32, 777, 32 * 300)
     assert K._prefill_has_decode_rows(4, 4, 1, 4 * 32)
