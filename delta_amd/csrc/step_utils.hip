@@ -39,12 +39,14 @@ __global__ void __launch_bounds__(kNormThreads)
   const float *pr = PART ? part + (int64_t)row * dim : nullptr;
   constexpr int kMaxChunks = 4;  // 8 elements per chunk -> dim <= 8192
   float hv[kMaxChunks][8];
+  u32x4 wv[kMaxChunks];  // loaded with the row, not behind its reduction (a memory round trip of the ~4 us)
   float ss = 0.f;
 #pragma unroll
   for (int k = 0; k < kMaxChunks; ++k) {
     const int c0 = (threadIdx.x + k * kNormThreads) * 8;
     if (c0 < dim) {
       const u32x4 a = ld128(xr + c0);
+      wv[k] = ld128(w + c0);
       u32x4 o;
       if (PART) {
         f32x4 pv[PS > 0 ? PS : 1][2];
@@ -102,7 +104,6 @@ __global__ void __launch_bounds__(kNormThreads)
   for (int k = 0; k < kMaxChunks; ++k) {
     const int c0 = (threadIdx.x + k * kNormThreads) * 8;
     if (c0 < dim) {
-      const u32x4 wv = ld128(w + c0);
       u32x4 o;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
@@ -113,7 +114,7 @@ __global__ void __launch_bounds__(kNormThreads)
         asm volatile("" : "+v"(m0), "+v"(m1));
         const float n0 = E::lo(E::from_float(m0));
         const float n1 = E::lo(E::from_float(m1));
-        o[q] = E::from_float(n0 * E::lo(wv[q])) | (E::from_float(n1 * E::hi(wv[q])) << 16);
+        o[q] = E::from_float(n0 * E::lo(wv[k][q])) | (E::from_float(n1 * E::hi(wv[k][q])) << 16);
       }
       st128(y + (int64_t)row * ys + c0, o);
     }
@@ -175,25 +176,52 @@ __device__ __forceinline__ void block_best(float &best, int &bi, float *s_val, i
 
 constexpr int kArgChunks = 32;
 
-template <int DT>
+// VEC: rows 16-byte aligned, 8 logits per load and four loads in flight (one 2-byte load per logit had
+// 64 rows of 151936 take 16 us); chunks are whole 16-byte units, the last one may end in a partial unit.
+template <int DT, bool VEC>
 __global__ void __launch_bounds__(256) argmax_chunk_kernel(const uint16_t *logits, int64_t stride, int cols,
                                                             float *ws_val, int *ws_idx) {
   using E = Elem<DT>;
   __shared__ float s_val[4];
   __shared__ int s_idx[4];
   const int r = blockIdx.y;
-  const int per = (cols + kArgChunks - 1) / kArgChunks;
+  const int per = ((cols + kArgChunks - 1) / kArgChunks + 7) / 8 * 8;
   const int c_beg = blockIdx.x * per;
   const int c_end = min(cols, c_beg + per);
   const uint16_t *row = logits + (int64_t)r * stride;
   float best = -INFINITY;
   int bi = 0x7fffffff;
-  for (int c = c_beg + threadIdx.x; c < c_end; c += 256) {
-    const float v = E::lo(row[c]);
-    if (bi == 0x7fffffff || better(v, c, best, bi)) {
-      best = v;
-      bi = c;
+  auto take = [&](float v, int c) {
+    if (!(v <= best) || bi == 0x7fffffff) {  // larger, a NaN on either side, or the first
+      if (bi == 0x7fffffff || better(v, c, best, bi)) {
+        best = v;
+        bi = c;
+      }
     }
+  };
+  if (VEC) {
+    constexpr int kLoads = 4, kStep = 256 * 8;
+    for (int c0 = c_beg + (int)threadIdx.x * 8; c0 < c_end; c0 += kLoads * kStep) {
+      u32x4 v[kLoads];
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i)
+        if (c0 + i * kStep + 8 <= c_end) v[i] = ld128(row + c0 + i * kStep);
+#pragma unroll
+      for (int i = 0; i < kLoads; ++i) {
+        const int c = c0 + i * kStep;
+        if (c + 8 <= c_end) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            take(E::lo(v[i][q]), c + 2 * q);
+            take(E::hi(v[i][q]), c + 2 * q + 1);
+          }
+        } else {
+          for (int e = c; e < c_end; ++e) take(E::lo(row[e]), e);
+        }
+      }
+    }
+  } else {
+    for (int c = c_beg + threadIdx.x; c < c_end; c += 256) take(E::lo(row[c]), c);
   }
   block_best(best, bi, s_val, s_idx);
   if (threadIdx.x == 0) {
@@ -245,12 +273,14 @@ extern "C" DELTA_EXPORT int delta_argmax_rows(const void *logits, int64_t row_st
   int *wi = (int *)((char *)workspace + (size_t)rows * kArgChunks * sizeof(float));
   hipStream_t st = (hipStream_t)stream;
   dim3 grid(kArgChunks, rows);
+  const bool vec = !((uintptr_t)logits & 15u) && row_stride % 8 == 0;
+  auto launch = [&](auto k) {
+    hipLaunchKernelGGL(k, grid, dim3(256), 0, st, (const uint16_t *)logits, row_stride, cols, wv, wi);
+  };
   if (dtype == DELTA_BF16)
-    hipLaunchKernelGGL(argmax_chunk_kernel<DELTA_BF16>, grid, dim3(256), 0, st, (const uint16_t *)logits,
-                       row_stride, cols, wv, wi);
+    vec ? launch(argmax_chunk_kernel<DELTA_BF16, true>) : launch(argmax_chunk_kernel<DELTA_BF16, false>);
   else
-    hipLaunchKernelGGL(argmax_chunk_kernel<DELTA_FP16>, grid, dim3(256), 0, st, (const uint16_t *)logits,
-                       row_stride, cols, wv, wi);
+    vec ? launch(argmax_chunk_kernel<DELTA_FP16, true>) : launch(argmax_chunk_kernel<DELTA_FP16, false>);
   int rc = check_launch("delta_argmax_rows");
   if (rc) return rc;
   hipLaunchKernelGGL(argmax_final_kernel, dim3(rows), dim3(64), 0, st, wv, wi, out, out_stride);

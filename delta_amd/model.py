@@ -218,6 +218,10 @@ def dense(x: Tensor, layer: nn.Linear) -> Tensor:
         rows = x.numel() // x.shape[-1]
         if rows <= _SKINNY_ROWS_ANY or w.numel() * w.element_size() <= _SKINNY_MAX_WEIGHT_BYTES:
             return K.gemm_skinny(x, w, layer.bias)
+    elif w.shape[0] >= _ROWS128_WIDE and w.shape[1] <= 2048 and K.gemm_rows128_ok(x, w):
+        rows = x.numel() // x.shape[-1]
+        if _ROWS32_MAX < rows <= 64 and K.gemm_rows128_splits(rows, *w.shape) == 1:
+            return K.gemm_rows128(x, w, layer.bias)
     return layer(x)
 
 
@@ -234,8 +238,10 @@ _ROWS32_MAX = 32
 # 32.1, w1|w3 65-73 vs 73 and 5).  It stays on hipBLASLt where that is faster: past 64 rows weights of
 # fewer than 8 M elements (the 1.5B wo: 8.5 vs 7.1, and the norm's partials come on top) and gate/up
 # launches of more than 256 blocks of 64 columns, a second pass over the CUs (Qwen2.5-7B w1|w3: 80-89
-# vs 72); wqkv and lm_head too, whose consumers sum no partials (14B wqkv unsplit 40 vs 33).
+# vs 72); wqkv and lm_head too, whose consumers sum no partials (14B wqkv unsplit 40 vs 33), but for
+# an lm_head of few features at up to 64 rows (1.5B, K = 1536: 100 vs 113; 8B, K = 4096: 212 vs 211).
 _ROWS128_MAX = 128
+_ROWS128_WIDE = 32768
 _ROWS128_MIN_WEIGHT = 8 << 20
 _ROWS128_GLU_MAX = 64 * 256
 
