@@ -355,8 +355,9 @@ class FeedForward(nn.Module):
     ``x @ w13.T``.  An engine set up for at most 128 rows per step re-lays it out row-major
     (``w13`` ``[2 * inter, dim]``, ``use_row_major_w13``): ``delta_gemm_skinny`` streams it faster
     still at <= 8 rows (Qwen2.5-7B, 4 rows: 41 vs 53 us) and ``delta_gemm_rows32_silu`` /
-    ``delta_gemm_rows128_silu`` fuse the SiLU-mul into the GEMM at 9-32 and 33-128 rows.  Checkpoints with separate ``w1`` /
-    ``w3`` (the reference's names, ``[inter, dim]`` each) are merged and transposed on load."""
+    ``delta_gemm_rows128_silu`` fuse the SiLU-mul into the GEMM at 9-32 and 33-128 rows.
+    Checkpoints with separate ``w1`` / ``w3`` (the reference's names, ``[inter, dim]`` each) are
+    merged on load, and a state saved in either layout loads into the other."""
 
     def __init__(self, config: ModelArgs) -> None:
         super().__init__()
@@ -366,14 +367,14 @@ class FeedForward(nn.Module):
         self._register_load_state_dict_pre_hook(self._merge_w1_w3)
 
     def _merge_w1_w3(self, state_dict, prefix, *args):
-        """Separate ``w1`` / ``w3`` weights load into the merged gate|up parameter in whichever
-        layout this module holds it (transposed ``w13_t`` or row-major ``w13``)."""
+        """Separate ``w1`` / ``w3`` weights, and a merged gate|up weight saved in the other layout, load
+        into whichever layout this module holds (transposed ``w13_t`` or row-major ``w13``)."""
+        mine, other = ("w13", "w13_t") if hasattr(self, "w13") else ("w13_t", "w13")
         if prefix + "w1.weight" in state_dict:
             w13 = torch.cat([state_dict.pop(prefix + "w1.weight"), state_dict.pop(prefix + "w3.weight")])
-            if hasattr(self, "w13"):
-                state_dict[prefix + "w13"] = w13
-            else:
-                state_dict[prefix + "w13_t"] = w13.t().contiguous()
+            state_dict[prefix + mine] = w13 if mine == "w13" else w13.t().contiguous()
+        elif prefix + other in state_dict and prefix + mine not in state_dict:
+            state_dict[prefix + mine] = state_dict.pop(prefix + other).t().contiguous()
 
     @torch.no_grad()
     def use_row_major_w13(self) -> None:

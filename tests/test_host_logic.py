@@ -211,6 +211,26 @@ def test_checkpoint_with_separate_projections_loads_every_parameter(tmp_path):
         LMBackend(device="cpu").load_model(path)
 
 
+@pytest.mark.parametrize("saved, held", [("w13_t", "w13"), ("w13", "w13_t"), ("w13", "w13"), ("w13_t", "w13_t")])
+def test_state_saved_in_either_gate_up_layout_loads_into_the_other(saved, held):
+    """An engine of up to 128 rows holds the gate|up weight row-major: states saved before (or by a
+    larger engine) carry it transposed, and the other way round."""
+    from delta_amd.model import build_random_model
+    src, dst = (build_random_model("tiny-test", "cpu", torch.bfloat16, seed=s) for s in (5, 6))
+    want = [layer.feed_forward.w13_t.detach().clone() for layer in src.layers]
+    for model, layout in ((src, saved), (dst, held)):
+        if layout == "w13":
+            for layer in model.layers:
+                layer.feed_forward.use_row_major_w13()
+    state = src.state_dict()
+    keys = list(state)
+    dst.load_state_dict(state, strict=True)
+    assert list(state) == keys
+    for layer, w in zip(dst.layers, want):
+        ff = layer.feed_forward
+        assert torch.equal(ff.w13.t() if held == "w13" else ff.w13_t, w)
+
+
 def test_qkv_bias_and_row_major_gate_up_merge_on_load():
     from delta_amd.model import build_random_model
     src = build_random_model("tiny-test", "cpu", torch.float32, seed=3, qkv_bias=True)
