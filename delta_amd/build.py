@@ -25,7 +25,7 @@ SOURCES = ["capi.hip", "paged_decode.hip", "page_score.hip", "page_select.hip",
 COMPILE_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "-fvisibility=hidden",
     "--offload-arch=gfx950",
-    # Packed fp32 instructions off (v_pk_{add,mul,fma}_f32 are avoided on this pool).
+    # Packed fp32 instructions off (v_pk_{add,mul,fma}_f32 have given wrong results).
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     "-Wno-unused-result",
 ]

@@ -52,10 +52,10 @@ template <bool STREAM = false>
 __device__ __forceinline__ void load_lds_1k(uint32_t lds, const void *base, uint32_t off) {
   if constexpr (STREAM)
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 nt" ::"s"(lds), "v"(off), "s"(base)
-                 : "memory");
+                 : "memory", "m0");
   else
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(off), "s"(base)
-                 : "memory");
+                 : "memory", "m0");
 }
 // At most N of the wave's vector loads outstanding, and its LDS reads done.
 template <int N>
