@@ -275,13 +275,19 @@ def paged_decode_scores(q: torch.Tensor, kv_cache: torch.Tensor, kv_indptr: torc
 
 def _prefill_has_decode_rows(tokens: int, batch: int, max_qo_len: int, pages: int) -> bool:
     """Whether a prompt step is likely to hold rows with one new token and a long cache: the rows but
-    the longest average under half its tokens (the row lengths themselves are on the device), and a row
-    holds 512 cached tokens or more on average.  One prefill block per kv head sweeps such a row alone
-    (31 rows of 1-8 k tokens beside a 777-token prompt: 207 us against 133 us with split decode units);
-    where no row has one token the two extra launches find nothing to do (~5 us)."""
-    if batch <= 0 or max_qo_len <= 0 or pages < 32 * batch:
+    the longest average under half its tokens (the row lengths themselves are on the device), and hold
+    1024 cached tokens or more on average (1344 below 16 rows).  One prefill block per kv head sweeps
+    such a row alone (31 rows of 1-8 k tokens beside a 777-token prompt: 207 us against 147 with split
+    decode units; 30 of 0.5-2.7 k beside 8 short prompts: 67 / 44; 5 of 0.5-2 k beside 100 tokens: 46 / 32),
+    but the two extra launches cost ~5 us: 5 rows of 0.5-1 k 28-30 / 33, 30 of them 45.8 / 46.5, 5 of
+    0.5-1.4 k beside prompts at 1000 tokens 44-46 / 48."""
+    if batch <= 0 or max_qo_len <= 0:
         return False
-    return max_qo_len == 1 or (batch > 1 and 2 * (tokens - max_qo_len) < (batch - 1) * max_qo_len)
+    long_pages = 64 if batch >= 16 else 84
+    if max_qo_len == 1:
+        return pages >= long_pages * batch
+    return (batch > 1 and 2 * (tokens - max_qo_len) < (batch - 1) * max_qo_len
+            and pages - (max_qo_len + 15) // 16 >= long_pages * (batch - 1))
 
 
 def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, qo_indptr: torch.Tensor,

@@ -129,8 +129,10 @@ def test_prefill_block_orders_match_a_row_at_a_time(lens):
 @torch.inference_mode()  # as the engine captures: torch's graph state must not change mode between captures
 def test_paged_prefill_takes_the_rows_path_where_it_should():
     assert K._prefill_has_decode_rows(808, 32, 777, 32 * 300)
-    assert K._prefill_has_decode_rows(4, 4, 1, 4 * 32)
-    assert not K._prefill_has_decode_rows(4, 4, 1, 4 * 32 - 1)     # short rows
+    assert K._prefill_has_decode_rows(4, 4, 1, 4 * 84)
+    assert not K._prefill_has_decode_rows(4, 4, 1, 4 * 84 - 1)     # short rows
+    assert K._prefill_has_decode_rows(131, 32, 100, 7 + 31 * 64)
+    assert not K._prefill_has_decode_rows(131, 32, 100, 6 + 31 * 64)
     assert not K._prefill_has_decode_rows(8192, 1, 8192, 513)      # one prompt
     assert not K._prefill_has_decode_rows(8 * 1024, 8, 1024, 8 * 65)  # equal prompts
     rows, hq, hkv, dtype = CASES["joins_g7_chunked"]
