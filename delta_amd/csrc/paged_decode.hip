@@ -1301,17 +1301,25 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
       R = 1;
     }
   } else if (small && (int64_t)batch * hkv >= 32) {
-    // Longer units (full attention of small batches): about 1024 one-wave blocks, at least 4 waves per
-    // CU, each storing its partial from registers; a ragged batch's units stay short.  Against 16-wave
-    // blocks, with the merge: 64 rows of 513 pages, 2 kv heads (8 splits) 109.5 -> 87.0 us (in a decode
-    // step 106 -> 84.5 without it); 8 rows of 1025 pages, 8 kv heads 99.0 -> 87; 16 rows of 129 pages,
-    // 8 kv heads 30.3 -> 29.0.  Fewer than 32 (row, kv head) pairs would need more than 32 splits, whose
-    // partials the merge pays for, and keep 16-wave blocks: with 4 waves the config-4 full attention (4
-    // rows of 4097 pages, 4 kv heads) is as fast alone (90.5 vs 92.8 us) but slower in a step (103 vs 90).
-    ns = ceil_div(1024, (int64_t)batch * hkv);
-    if (ns < ceil_div(max_pages, kMaxChunk)) ns = ceil_div(max_pages, kMaxChunk);
-    ch = ceil_div(max_pages, ns);
-    R = 1;
+    // Longer units (full attention of small batches).  Where about 1024 blocks leave a unit at most 16
+    // pages: one-wave units that store their partials from registers (50 rows of 133 pages, 2 kv heads:
+    // 32.7 -> 24.9 us with the merge; 31 of 69, 8: 32.1 -> 28.6; 30 of 132, 4: 33.4 -> 29.0).  Not past that:
+    // max_pages is often a slot's size, and rows far below it would be one wave's serial sweep (64 rows of
+    // 130 pages, 2 kv heads, max_pages 1153, units of 116: 86 us against 53).  Then 8-wave units of 64 pages
+    // instead of 16-wave ones of 128, for 2 kv heads or up to 64 pairs: those 64 rows of 130 pages 53 -> 39,
+    // of 514 pages (max_pages 517) 110 -> 95, of 1026 190 -> 183; 8 rows of 1000 pages, 8 kv heads 91 -> 87,
+    // of 130 64 -> 50.  More pairs of more heads keep 128 (30 rows of 1000 pages, 4 kv heads 162 / 169 with
+    // 64; 16 of 64, 8 kv heads 22 / 29), and so do fewer than 32 pairs and very long rows (their partials).
+    const int64_t pairs = (int64_t)batch * hkv, fine = ceil_div(1024, pairs);
+    if (ceil_div(max_pages, fine) <= 16) {
+      ns = fine;
+      ch = ceil_div(max_pages, ns);
+      R = 1;
+    } else if ((hkv <= 2 || pairs <= 64) && pairs * max_pages <= kHeadMajorPageHeads) {
+      ns = ceil_div(max_pages, ch < 64 ? ch : (int64_t)64);
+      if (ch > 64) ch = 64;
+      R = 8;
+    }
   }
   *nsplit = (int)ns;
   *waves = h * R;
