@@ -1292,33 +1292,19 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
   // (an unsplit launch keeps its blocks: no merge launch), each wave
   // storing its partial from registers with no closing block merge (config-2 subset 17.4 -> 16.6
   // us; at config 4, 16 -> 64 splits, the merge's 4x partials cost more than the block merge
-  // saves: 13.6 -> 14.2 us).
+  // saves: 13.6 -> 14.2 us).  Others keep 16 waves (the config-4 full attention, 128-page units:
+  // with 4 waves its full-cache engine step ran 5.4-5.6 -> 5.9-6.0 ms, though a launch timed alone
+  // was unchanged).  One-wave units of up to 16 pages and 8-wave units of 64 were measured over 12
+  // (rows, kv heads), 40-2100 max_pages and rows of 10-100 % of it: faster at most of them (50 rows of
+  // 133 pages, 2 kv heads: 32.6 -> 25.4 us), but 1.1-1.4 times as long at a third (rows of 13 pages
+  // under max_pages 133: 12.9 -> 16.1; 64 rows of 66 under 264: 23.2 -> 32.1; 8 rows of 264, 8 kv heads:
+  // 29.8 -> 36.1), and max_pages says nothing about the rows' lengths, so no rule on it can tell.
   if (small && ceil_div(ch, (int64_t)kHeadMajorWaves) <= 8) {
     R = kHeadMajorWaves;
     if (ns > 1 && ns * kHeadMajorWaves <= 16 && ns * kHeadMajorWaves <= max_pages) {
       ns *= kHeadMajorWaves;
       ch = ceil_div(max_pages, ns);
       R = 1;
-    }
-  } else if (small && (int64_t)batch * hkv >= 32) {
-    // Longer units (full attention of small batches).  Where about 1024 blocks leave a unit at most 16
-    // pages: one-wave units that store their partials from registers (50 rows of 133 pages, 2 kv heads:
-    // 32.7 -> 24.9 us with the merge; 31 of 69, 8: 32.1 -> 28.6; 30 of 132, 4: 33.4 -> 29.0).  Not past that:
-    // max_pages is often a slot's size, and rows far below it would be one wave's serial sweep (64 rows of
-    // 130 pages, 2 kv heads, max_pages 1153, units of 116: 86 us against 53).  Then 8-wave units of 64 pages
-    // instead of 16-wave ones of 128, for 2 kv heads or up to 64 pairs: those 64 rows of 130 pages 53 -> 39,
-    // of 514 pages (max_pages 517) 110 -> 95, of 1026 190 -> 183; 8 rows of 1000 pages, 8 kv heads 91 -> 87,
-    // of 130 64 -> 50.  More pairs of more heads keep 128 (30 rows of 1000 pages, 4 kv heads 162 / 169 with
-    // 64; 16 of 64, 8 kv heads 22 / 29), and so do fewer than 32 pairs and very long rows (their partials).
-    const int64_t pairs = (int64_t)batch * hkv, fine = ceil_div(1024, pairs);
-    if (ceil_div(max_pages, fine) <= 16) {
-      ns = fine;
-      ch = ceil_div(max_pages, ns);
-      R = 1;
-    } else if ((hkv <= 2 || pairs <= 64) && pairs * max_pages <= kHeadMajorPageHeads) {
-      ns = ceil_div(max_pages, ch < 64 ? ch : (int64_t)64);
-      if (ch > 64) ch = 64;
-      R = 8;
     }
   }
   *nsplit = (int)ns;

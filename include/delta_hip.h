@@ -66,8 +66,8 @@ int delta_abi_version(void);
 
 /* Most split-K work units a row is cut into for this shape (1 = unsplit).  A
  * split launch cuts each row into clamp(ceil(pages_b / chunk), 1, splits)
- * units of at most 128 pages and packs them row by row, so ragged rows cost in
- * proportion to their pages.  Depends only on its arguments, so a value
+ * units of at most 128 pages (136 where that saves a unit of 8) and packs
+ * them row by row, so ragged rows cost in proportion to their pages.  Depends only on its arguments, so a value
  * computed at graph capture stays valid for every replay.  max_pages_per_row
  * is the planned maximum of pages_b (a longer row is still covered whole: its
  * last unit takes the remainder). */

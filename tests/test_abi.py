@@ -83,6 +83,34 @@ def test_queries_without_gpu(lib):
     assert lib.delta_page_score_kv_workspace_bytes(1024, 32, 8, 2048) == 1024 * 32 * 4
 
 
+@pytest.mark.parametrize("batch,hq,hkv", [(16, 12, 2), (64, 12, 2), (100, 12, 2), (15, 28, 4), (8, 32, 8), (31, 32, 8)])
+def test_a_workspace_kept_for_long_rows_serves_shorter_ones(lib, batch, hq, hkv):
+    """A server sizes its workspace once, for its largest max_pages: launches planned for fewer pages fit
+    it.  32-255 (row, kv head) pairs, where a launch of few pages must not be cut into more units than one
+    of many (one-wave units of up to 16 pages were: 32 splits at 500 pages, 19 at 1153)."""
+    need = [lib.delta_paged_decode_workspace_bytes(batch, hq, hkv, n) for n in range(1, 2101)]
+    for kept in (1153, 2100):
+        assert max(need[:kept]) == need[kept - 1]
+
+
+def test_small_attention_plans(lib):
+    """Attention launches of 32-255 pairs: about 256 blocks, units of at most 128 pages.  Finer units were
+    faster for full rows and slower for rows far below max_pages, which the plan cannot see.  (The query
+    is the larger of this plan and the dump launch's, here the first.)"""
+    for (batch, hkv, pages), splits in {(100, 2, 69): 2, (60, 4, 69): 2, (100, 2, 1153): 10, (60, 4, 2100): 17}.items():
+        assert lib.delta_decode_num_splits(batch, hkv, pages) == max(splits, _dump_splits(batch, hkv, pages))
+
+
+def _dump_splits(batch, hkv, pages):
+    """Splits of a page-major dump launch: 4096 waves in 16-wave blocks, >= 2 pages a wave, units of at most
+    128 pages (136 where that saves a unit of 8)."""
+    ns = max(1, min(-(-4096 // (batch * 16)), pages // (2 * (16 // hkv))))
+    if ns > 1 and -(-pages // ns) > 128:
+        ns = -(-pages // 128)
+        ns -= ns > 1 and pages - (ns - 1) * 128 <= 8
+    return ns
+
+
 def test_argument_errors_reported_without_launch(lib):
     from delta_amd import _lib
     # head_dim 64 is rejected before any launch; the message is kept per thread

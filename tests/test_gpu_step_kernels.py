@@ -29,16 +29,16 @@ def test_argmax_rows_vector_and_scalar_paths(dtype, rows, cols, stride):
 
 
 @pytest.mark.parametrize("batch,hq,hkv,lens", [
-    (64, 12, 2, [8200] * 64),                            # 128 pairs: 8-wave units of 64 pages, a rest of one
-    (8, 32, 8, [16384 - 900 * i for i in range(8)]),     # 64 pairs, 64-page units, ragged
+    (64, 12, 2, [8200] * 64),                            # 128 pairs, 128-page units, a rest of one page
+    (8, 32, 8, [16384 - 900 * i for i in range(8)]),     # 64 pairs, ragged
     (4, 32, 8, [700, 16, 5000, 1]),                      # 32 pairs, most rows one unit
-    (15, 28, 4, [33 * 16 + i for i in range(15)]),       # 60 pairs, one-wave units of 2 pages, partial last pages
-    (31, 16, 8, [3000] * 31),                            # 248 pairs, 16-wave units
-    (31, 16, 8, [1279] * 30 + [17]),                     # 248 pairs, one-wave units of 16 pages
+    (15, 28, 4, [33 * 16 + i for i in range(15)]),       # 60 pairs, 4-wave units, partial last pages
+    (31, 16, 8, [3000] * 31),                            # 248 pairs, two units of 94 pages
+    (31, 16, 8, [1279] * 30 + [17]),                     # 248 pairs, two units of 40 pages
 ])
 def test_small_attention_plans_match_the_dump_launch(batch, hq, hkv, lens):
-    """Attention launches of 32-255 (row, kv head) pairs split into one-wave, 8-wave or 16-wave units; the dump launch of the
-    same rows splits page-major.  Both round P to bf16 from sums in another order: 2e-2, the attention
+    """Attention launches of 32-255 (row, kv head) pairs split into units of one kv head; the dump launch of
+    the same rows splits page-major.  Both round P to bf16 from sums in another order: 2e-2, the attention
     tolerance; lse in fp32."""
     c = make_case(batch=batch, hq=hq, hkv=hkv, kv_lens=lens, seed=batch, k=4, L=2).to(DEV)
     args = (c.q, c.kv_cache, c.kv_indptr, c.kv_indices, c.kv_last_page_len)
