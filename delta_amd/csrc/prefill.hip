@@ -45,12 +45,9 @@
 //         O[row l%32][d = 32 dt + 8 (i / 4) + 4 (l / 32) + i % 4].
 // LDS tiles: 64 rows of 256 bytes, 16-byte chunks swizzled by row so that the fragment reads cover
 // the banks once (see the step loads).  Page ids come by scalar loads, a step ahead.
-// Blocks run heaviest first (the last query tiles attend the most tokens), the kv head fastest, so
-// with 8 kv heads the blocks of one head land on the same XCD (blocks go to the XCDs round robin)
-// and share its L2 for that head's K/V.  Up to 6144 kv tokens all rows run together, past that in groups
-// of about 3072: one row at a time leaves the last rows' heavy tiles to the end (8 prompts of 37-1500,
-// 5.5 k tokens: 71.4 vs 64.5 us), too many rows at once overflow the L2 (16 prompts of 512: all 93.3 us,
-// 8 rows 73.8, 4 rows 65.9, one 69.4).  No merge.
+// Blocks run heaviest first (the last query tiles attend the most tokens; see BlockOrder), the kv head
+// fastest, so with 8 kv heads the blocks of one head land on the same XCD (blocks go to the XCDs round
+// robin) and share its L2 for that head's K/V.  No merge.
 #include "delta_common.h"
 
 namespace delta {
@@ -68,8 +65,24 @@ constexpr int kSub = 2;         // 32-token sub-tiles per step
 constexpr int kKvStep = 32 * kSub;  // kv tokens per step
 constexpr int kPgStep = kKvStep / 16;  // pages per step
 constexpr int kWideQo = 4096;   // longest prompt from which blocks hold 8 waves
-constexpr int kGroupTokens = 3072;  // kv tokens of the rows whose blocks run together (see the block order)
 constexpr int kTileB = kKvStep * 256;  // bytes of a step's K (or V) tile: 64 rows of 256 bytes
+
+// Order of a kv head's blocks (find_tile).  A slot of the grid without a tile costs a launched block that
+// holds LDS for a microsecond, and many of them among the others hold those back (prompts of 4096 and
+// 1500 tokens, the shorter one's missing tiles launched between the longer one's: 232 us, packed 165;
+// prompts of 300 beside 100 decoding rows, a row's slots together: 103, packed 77), so the blocks that
+// exist come first:
+//   kByTile, few rows: the last tiles of all rows first (they attend the most tokens), down to the rows'
+//     first ones.  A row at a time leaves the last rows' heavy tiles to the end of the launch (us by tile / by
+//     row: 8 prompts of 37-1500, 2 kv heads 42.6 / 55.7, 8 kv heads 99.6 / 102; 4 of 2048, 2 kv heads
+//     71.7 / 88.4; 12 of 1000, 2 kv heads 63.7 / 68.1).
+//   kByRow, more rows: a row's last tile first, then the next row.  What runs together shares few rows' K
+//     and V in the L2 (16 prompts of 512, 8 kv heads 79.6 / 71.5; 32 of 64-256 40.8 / 36.4; 64 of 128
+//     66.0 / 52.3).
+//   kBySlot, one row or no more slots than the CUs hold at once: nothing to order, no search in front (100
+//     prompts of 30, 2 kv heads 11.8 / 12.2 by row).
+enum BlockOrder { kBySlot = 0, kByRow = 1, kByTile = 2 };
+constexpr int kByTileRows = 12;
 
 struct PrefillArgs {
   const uint16_t *q;
@@ -86,6 +99,8 @@ struct PrefillArgs {
   float *lse;
   int batch, hq, hkv;
   int skip_single;  // rows of one query token are run_decode_rows'
+  int row_tiles;    // the most tiles a row has (of max_qo_len tokens)
+  int order;        // of the blocks: kBySlot, kByRow, kByTile
   float sm_scale;
 };
 
@@ -136,6 +151,77 @@ __device__ __forceinline__ float halves_sum(float v) {
   return __uint_as_float(x[0]) + __uint_as_float(x[1]);
 }
 
+// Row and tile (BT query tokens) of block u of a kv head; false past the last one.  Only the device knows
+// the rows' lengths, so the grid has batch * row_tiles slots.
+template <int BT>
+__device__ __forceinline__ bool find_tile(const PrefillArgs &a, int u, int lane, int *row, int *tile) {
+  auto tiles_of = [&](int r) {
+    if (r >= a.batch) return 0;
+    const int qn = a.qo_indptr[r + 1] - a.qo_indptr[r];
+    if (qn <= 0 || (a.skip_single && qn == 1)) return 0;
+    const int n = (qn + BT - 1) / BT;
+    return n < a.row_tiles ? n : a.row_tiles;
+  };
+  if (a.order == kBySlot) {
+    *row = u / a.row_tiles;
+    *tile = a.row_tiles - 1 - (u - *row * a.row_tiles);
+    return *row < a.batch && *tile < tiles_of(*row);
+  }
+  if (a.order == kByTile) {  // batch <= 64, row_tiles <= 32 * 64
+    // Lane l counts the blocks from tile t_l on, sum over the rows of max(0, n_r - t_l), for 64 t at
+    // once (more tiles: coarse, then fine).
+    const int n = tiles_of(lane);
+    auto blocks_from = [&](int t) {
+      int s = 0;
+      for (int r = 0; r < a.batch; ++r) {
+        const int d = __builtin_amdgcn_readlane(n, r) - t;
+        s += d > 0 ? d : 0;
+      }
+      return s;
+    };
+    const int step = (a.row_tiles + 63) / 64;
+    int t0 = 0;
+    if (step > 1) {
+      const uint64_t m = __ballot(blocks_from(lane * step) > u);
+      if (m == 0) return false;
+      t0 = (__popcll(m) - 1) * step;
+    }
+    const int s = blocks_from(t0 + lane);
+    const uint64_t m = __ballot(s > u);
+    if (m == 0) return false;
+    const int k = __popcll(m) - 1;  // 63 only if row_tiles = 64, whose tile 64 has no blocks
+    const int above = k < 63 ? __builtin_amdgcn_readlane(s, k < 63 ? k + 1 : 63) : 0;
+    const int t = t0 + k;
+    // The rows rotate by tile: blocks go to the XCDs round robin, and with fewer than 8 kv heads a fixed
+    // order would give an XCD all tiles of the same rows.
+    const uint64_t has = __ballot(n > t);
+    const int i = (u - above + t) % __popcll(has);
+    const bool mine = n > t && __popcll(has & ((1ull << lane) - 1)) == i;
+    *row = __builtin_ctzll(__ballot(mine));
+    *tile = t;
+    return true;
+  }
+  int base = 0;
+  for (int r0 = 0; r0 < a.batch; r0 += 64) {
+    const int n = tiles_of(r0 + lane);
+    int incl = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(incl, off, 64);
+      if (lane >= off) incl += v;
+    }
+    const uint64_t m = __ballot(base + incl > u);
+    if (m != 0) {
+      const int l = __builtin_ctzll(m);
+      *row = r0 + l;
+      *tile = base + __builtin_amdgcn_readlane(incl, l) - 1 - u;
+      return true;
+    }
+    base += __builtin_amdgcn_readlane(incl, 63);
+  }
+  return false;
+}
+
 template <int DT, int G, int PW>
 __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a) {
 #pragma clang fp contract(off)
@@ -152,16 +238,12 @@ __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a
 
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int hl = lane >> 5, n = lane & 31;
-  // Blocks run in groups of gridDim.x / hkv rows (blockIdx.z).  Within a group the rows rotate by tile: blocks go to the XCDs round robin, and with fewer
-  // than 8 kv heads a fixed order would give an XCD all tiles of the same rows.
-  const int h = (int)blockIdx.x % a.hkv, grp_rows = (int)gridDim.x / a.hkv;
-  const int b = (int)blockIdx.z * grp_rows + (int)((blockIdx.x / a.hkv + blockIdx.y) % grp_rows);
-  if (b >= a.batch) return;
+  const int h = blockIdx.x;
+  int b, tile;
+  if (!find_tile<BT>(a, (int)(blockIdx.z * gridDim.y + blockIdx.y), lane, &b, &tile)) return;  // whole block
   const int64_t q0 = a.qo_indptr[b], q1 = a.qo_indptr[b + 1];
-  const int qn = q1 > q0 ? (int)(q1 - q0) : 0;
-  const int tile = (int)gridDim.y - 1 - (int)blockIdx.y;
+  const int qn = (int)(q1 - q0);
   const int btok0 = tile * BT;
-  if (btok0 >= qn || (a.skip_single && qn == 1)) return;  // whole block
   // The wave's first query token, read as a scalar: the compiler cannot see that wave (from the
   // thread index) is uniform, and with tok0 scalar the wave's step count and its diagonal test
   // (full / masked step) become scalar branches (8192-token prompt 594 -> 569-585 us).
@@ -461,13 +543,16 @@ __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a
 }
 
 template <int DT, int G>
-void launch_prefill_g(const PrefillArgs &a, int max_qo, hipStream_t stream) {
+void launch_prefill_g(PrefillArgs a, int max_qo, hipStream_t stream) {
   const bool wide = max_qo >= kWideQo;
   const int bt = 32 / G * (wide ? 8 : 4);
-  const int64_t kv_tokens = a.kv_indices_len * kPageSize;
-  int64_t rows = kv_tokens <= 2 * kGroupTokens ? a.batch : kGroupTokens * (int64_t)a.batch / kv_tokens;
-  rows = rows < 1 ? 1 : (rows > a.batch ? a.batch : rows);
-  const dim3 grid((unsigned)(a.hkv * rows), (unsigned)ceil_div(max_qo, bt), (unsigned)ceil_div(a.batch, rows));
+  a.row_tiles = (int)ceil_div(max_qo, bt);
+  const int64_t slots = (int64_t)a.batch * a.row_tiles;
+  a.order = a.batch == 1 || slots * a.hkv <= (wide ? 256 : 512) ? kBySlot
+            : a.batch <= kByTileRows && a.row_tiles <= 32 * 64  ? kByTile
+                                                                : kByRow;
+  const int64_t y = slots < 32768 ? slots : 32768;
+  const dim3 grid((unsigned)a.hkv, (unsigned)y, (unsigned)ceil_div(slots, y));
   if (wide)
     hipLaunchKernelGGL((paged_prefill_kernel<DT, G, 8>), grid, dim3(512), 0, stream, a);
   else

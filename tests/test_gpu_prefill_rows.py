@@ -111,10 +111,13 @@ def test_prefill_rows_zero_length_and_invalid_pages():
     assert torch.all(o1[301] == 0) and torch.all(l1[301] == float("-inf"))
 
 
-@pytest.mark.parametrize("lens", [[5000, 4100], [64] * 40, [3, 700, 64, 65, 1, 2000, 511, 4095]])
+@pytest.mark.parametrize("lens", [[5000, 4100], [64] * 40, [3, 700, 64, 65, 1, 2000, 511, 4095],
+                                  [1024, 1, 1009, 16],                    # by tile, 64 tiles a row
+                                  [40] * 63 + [900, 17, 16] + [5] * 70,   # by row, past 64 and 128 rows
+                                  [17] * 12, [17] * 13, [1] * 64])        # few slots: by slot
 def test_prefill_block_orders_match_a_row_at_a_time(lens):
-    """8-wave blocks (4096 tokens and more), 4-wave blocks, rows in one group and in several: each row
-    equals the launch of that row alone, bit for bit where both use the same block size."""
+    """8-wave blocks (4096 tokens and more), 4-wave blocks, blocks by tile (up to 12 rows), by row and by
+    slot: each row equals the launch of that row alone, bit for bit where both use the same block size."""
     c = build([(n, n) for n in lens], 28, 4, torch.bfloat16, seed=sum(lens))
     o, lse = launch(c, False, max(lens))
     qo, ptr = c["qo"].tolist(), c["ptr"].tolist()
