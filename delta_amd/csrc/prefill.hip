@@ -12,7 +12,7 @@
 // two 32-token sub-tiles) up to its last token's position: each step's K and V (16 KiB each for
 // one head) go from global memory straight to LDS (global_load_lds: no registers, no LDS store
 // instructions) and are read by every wave.
-//   PW = 8 (prompts of 4096 tokens and more): one block per CU, four step buffers.  Waves 0-3 run each
+//   PW = 8 (long prompts, see wide_blocks): one block per CU, four step buffers.  Waves 0-3 run each
 //     step whole; waves 4-7, the second wave of each SIMD, run half a step behind (P.V of the
 //     previous step, then S and softmax of this one), so the two waves of a SIMD are not both in
 //     their softmax at once.  Steps are loaded two ahead.
@@ -64,7 +64,6 @@ namespace {
 constexpr int kSub = 2;         // 32-token sub-tiles per step
 constexpr int kKvStep = 32 * kSub;  // kv tokens per step
 constexpr int kPgStep = kKvStep / 16;  // pages per step
-constexpr int kWideQo = 4096;   // longest prompt from which blocks hold 8 waves
 constexpr int kTileB = kKvStep * 256;  // bytes of a step's K (or V) tile: 64 rows of 256 bytes
 
 // Order of a kv head's blocks (find_tile).  A slot of the grid without a tile costs a launched block that
@@ -542,9 +541,24 @@ __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a
   }
 }
 
+// Whether blocks hold 8 waves instead of 4 (bt4 query tokens).  Where CUs would be left without a block, 4
+// waves spread a prompt over twice as many; where the chip is full anyway, 8 waves run a step faster (loads
+// two steps ahead, P.V of one wave under the softmax of the other).
+bool wide_blocks(int batch, int hkv, int bt4, int max_qo) {
+  // The longest prompt alone is 850 4-wave blocks, nearly two rounds over the chip's 512.  us for 8 / 4
+  // waves, 8 kv heads of 4 q heads: 3000 tokens (752 blocks) 88.9 / 86.0, 3200 (800) 94.1 / 93.3, 3500 (880)
+  // 103.5 / 111, 4000 (1000) 131 / 142, 8192 (2048) 513 / 541; 2 kv heads of 6: 4096 (410) 105.5 / 94.6,
+  // 6500 (650) 172 / 165, 8192 (820) 231.5 / 230, 16384 (1640) 833 / 849.
+  if (hkv * ceil_div(max_qo, bt4) >= 850) return true;
+  // Prompts of one 8-wave block or two 4-wave ones, and the latter no longer fit one to a CU: 60 prompts
+  // of 20, 4 kv heads of 7 (240 / 480 blocks) 10.2 / 12.6 us; 100 of 30, 2 of 6 (200 / 400) 10.9 / 11.8.
+  const int64_t blocks = (int64_t)batch * hkv;
+  return max_qo > bt4 && max_qo <= 2 * bt4 && blocks <= 256 && 2 * blocks > 256;
+}
+
 template <int DT, int G>
 void launch_prefill_g(PrefillArgs a, int max_qo, hipStream_t stream) {
-  const bool wide = max_qo >= kWideQo;
+  const bool wide = wide_blocks(a.batch, a.hkv, 32 / G * 4, max_qo);
   const int bt = 32 / G * (wide ? 8 : 4);
   a.row_tiles = (int)ceil_div(max_qo, bt);
   const int64_t slots = (int64_t)a.batch * a.row_tiles;
