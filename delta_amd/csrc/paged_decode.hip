@@ -57,6 +57,7 @@ struct DecodeArgs {
   int64_t kv_indices_len;
   const int32_t *last_page_len;
   const int32_t *q_rows;  // ROWS launches: query-token CSR; only rows of exactly one token take part
+  int full_slots;         // ROWS launches: slots of full units (see part_slot)
   uint16_t *o;
   int64_t o_stride_b, o_stride_h;
   float *lse;
@@ -149,13 +150,22 @@ typedef __attribute__((address_space(3))) s4_t lds_s4_t;
 // Work units of a split launch: row b has units_of(b) = clamp(ceil(pages_b / chunk), 1,
 // nsplit) of them (its last unit takes any pages past units * chunk, so a row longer than the
 // planned maximum is still covered), numbered row by row.
-// (ROWS: a row of another token count has one unit, which exits.)
+// (ROWS: a row of another token count has one unit, which exits; the others as many as their pages need.)
 template <bool ROWS = false>
 __device__ __forceinline__ int units_of(const DecodeArgs &a, int b) {
   if (ROWS && a.q_rows[b + 1] - a.q_rows[b] != 1) return 1;
   const RowInfo r = row_info(a, b);
   const int n = (r.np + a.chunk - 1) / a.chunk;
-  return n < 1 ? 1 : (n > a.nsplit ? a.nsplit : n);
+  return n < 1 ? 1 : (!ROWS && n > a.nsplit ? a.nsplit : n);
+}
+
+// Partial slot of a unit.  ROWS: a row's full units sit from its first page / chunk on (its next row starts
+// at least as many chunks later, rounded down), its last one past all of those, at full_slots + row, so the
+// slots are as many as the pages need, however they are spread over the rows.
+template <bool ROWS>
+__device__ __forceinline__ int64_t part_slot(const DecodeArgs &a, int b, int64_t p0, int split, int nu) {
+  if (ROWS) return split < nu - 1 ? p0 / a.chunk + split : (int64_t)a.full_slots + b;
+  return (int64_t)b * a.nsplit + split;
 }
 
 // Row of block y of an unsplit head-major launch whose (row, kv head) blocks outnumber the CUs.
@@ -353,11 +363,10 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
   const int c = lane >> 4;
   const int t = lane & 15;
 
-  int b, split = 0, j0 = 0, j1;
+  int b, split = 0, nu = 1, j0 = 0, j1;
   RowInfo ri;
   const int unit = blockIdx.x;
   if (a.nsplit > 1) {
-    int nu;
     if (a.direct) {
       // Every row owns nsplit block slots: the row is known from the block index, so its bounds,
       // q and page ids load with no scan before them; slots past the row's units exit.
@@ -389,7 +398,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
   }
   // A split launch's partial slot (row, split), and whether this is the row's first split;
   // both wave-uniform, so kept in scalar registers across the page loop.
-  const int pslot = uniform(b * a.nsplit + split);
+  const int pslot = uniform((int)part_slot<ROWS>(a, b, ri.p0, split, nu));
   const bool split0 = uniform(split) == 0;
   // (ROPE) The append CSR's row bounds, requested with the row's own bounds: the slot's page
   // id below then needs no round trip of its own before the page stream starts.  Scalar loads:
@@ -1017,7 +1026,8 @@ __global__ void __launch_bounds__(kMaxWaves * 64) paged_decode_plan_tokmax_kerne
 // group q merges the batches of 16 splits that start at 16 q, 16 (q + ngrp), ..., and the
 // groups' sums then combine through LDS, so up to 64 splits cost one round of loads.  Partials
 // sit at (row, split), so each group's first batch issues its loads with the row bounds, not
-// after them (splits the row does not have weigh nothing).
+// after them (splits the row does not have weigh nothing).  ROWS: the slots follow from the row bounds;
+// past the row's units its last one's slot is read.
 template <int DT, bool ROWS>
 __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(DecodeArgs a, int G) {
   using E = Elem<DT>;
@@ -1033,9 +1043,9 @@ __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(D
     orow = a.q_rows[b];
     if (a.q_rows[b + 1] - orow != 1) return;  // whole block
   }
-  const int nu = units_of(a, b);
-  const int64_t stride = (int64_t)a.hkv * G;  // partial rows per split
-  const int64_t p0 = ((int64_t)b * a.nsplit * a.hkv + h) * G + g;
+  const int nu = units_of<ROWS>(a, b);
+  const int64_t first_page = ROWS ? row_info(a, b).p0 : 0;
+  const int64_t stride = (int64_t)a.hkv * G;  // partial rows per slot
   // Batches of 16 splits whose loads all issue together (weight 0 past the row's last split;
   // a group's first batch reads min(16, nsplit - 16 q) slots regardless of the row's count); the
   // running sums move to a new maximum between batches.
@@ -1044,7 +1054,7 @@ __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(D
     float mv[16], lv[16], av[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
-      const int64_t pidx = p0 + (int64_t)(s0 + (i < lim ? i : 0)) * stride;
+      const int64_t pidx = part_slot<ROWS>(a, b, first_page, s0 + (i < lim ? i : 0), nu) * stride + (int64_t)h * G + g;
       mv[i] = a.part_ml[pidx * 2];
       lv[i] = a.part_ml[pidx * 2 + 1];
       av[i] = a.part_acc[pidx * kHeadDim + dd];
@@ -1068,7 +1078,7 @@ __global__ void __launch_bounds__(kMergeGroups * kHeadDim) decode_merge_kernel(D
     M = cm;
   };
   const int first = 16 * grp;  // < nsplit: merge_groups gives no group past the last split
-  merge16(first, a.nsplit - first < 16 ? a.nsplit - first : 16);
+  merge16(first, !ROWS && a.nsplit - first < 16 ? a.nsplit - first : 16);
   for (int s0 = first + 16 * ngrp; s0 < nu; s0 += 16 * ngrp) merge16(s0, nu - s0);
   if (ngrp > 1) {
     if (dd == 0) {
@@ -1506,25 +1516,23 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h, const void
 
 // The rows of exactly one query token of a prompt step (delta_paged_prefill_rows): decode attention of
 // those rows over packed head-major work units of 4-wave blocks, then the merge.  Row lengths are only
-// on the device; the host knows the pages of all rows together, so a unit holds what brings the launch to
-// about 1024 blocks, 16-128 pages (4-32 per wave), and a row has at most the units of four times the
-// average length (16 at least, 128 at most; a longer row's last unit takes the rest): the merge reads a
-// row's first 16 slots per group whether used or not (32 rows, 7 units each: 64 slots 10.5 us).
-void decode_rows_plan(int batch, int hkv, int64_t pages, int *nsplit, int *chunk) {
+// on the device; the host knows the pages of these rows together, so a unit holds what brings the launch to
+// about 1024 blocks, 16-128 pages (4-32 per wave).  A row has all the units its pages need (with at most
+// four times the average row's, its last unit took the rest: a row of 4063 pages beside 30 of 7 and a prompt
+// of 50 tokens, 8 kv heads, 668 us against 84).  Units of at least 1 / 1024 of all cached pages keep the
+// partials of any step to 1025 + batch slots.
+constexpr int64_t kRowsFullSlots = 1024;
+int decode_rows_chunk(int hkv, int64_t pages, int64_t kv_indices_len) {
   int64_t ch = ceil_div(pages * hkv, 1024);
   ch = ch < 16 ? 16 : (ch > kMaxChunk ? kMaxChunk : ch);
-  int64_t cap = 128;
-  int64_t ns = ceil_div(pages, ch);
-  const int64_t fit = 4 * ceil_div(ceil_div(pages, batch), ch);  // rows of four times the average length
-  cap = fit < 16 ? 16 : (fit < cap ? fit : cap);
-  *nsplit = (int)(ns < 2 ? 2 : (ns > cap ? cap : ns));
-  *chunk = (int)ch;
+  const int64_t least = ceil_div(kv_indices_len, kRowsFullSlots);
+  return (int)(ch > least ? ch : least);
 }
 
-size_t decode_rows_workspace_bytes(int batch, int hq, int hkv, int64_t pages) {
-  int ns, ch;
-  decode_rows_plan(batch, hkv, pages, &ns, &ch);
-  return decode_workspace_bytes(batch, hq, ns, true);
+// Enough for any step of at most this batch and kv_indices_len.
+size_t decode_rows_workspace_bytes(int batch, int hq, int64_t kv_indices_len) {
+  const int64_t full = kv_indices_len / 16 < kRowsFullSlots ? kv_indices_len / 16 : kRowsFullSlots;
+  return ((size_t)(full + 1 + batch) * hq * (kHeadDim + 2) * sizeof(float) + 255) & ~(size_t)255;
 }
 
 namespace {
@@ -1550,12 +1558,13 @@ void launch_decode_rows(const DecodeArgs &a, int G, int units, hipStream_t strea
 }
 }  // namespace
 
-// Arguments as delta_paged_prefill, checked there; workspace of decode_rows_workspace_bytes, 256-byte aligned.
+// Arguments as delta_paged_prefill, checked there; `rows` rows of one token hold `pages` pages (for the plan
+// only); workspace of decode_rows_workspace_bytes, 256-byte aligned.
 int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache, int64_t num_pages,
                     const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices,
                     int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o, int64_t o_stride_t,
                     int64_t o_stride_h, float *lse, int batch, int hq, int hkv, int dtype, float sm_scale,
-                    void *workspace, hipStream_t stream, const char *who) {
+                    int rows, int64_t pages, void *workspace, hipStream_t stream, const char *who) {
   DecodeArgs a = {};
   a.q = (const uint16_t *)q;
   a.q_stride_b = q_stride_t;
@@ -1576,9 +1585,13 @@ int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const
   a.hkv = hkv;
   a.hb = 1;
   a.sm_scale = sm_scale;
-  decode_rows_plan(batch, hkv, kv_indices_len, &a.nsplit, &a.chunk);
+  a.chunk = decode_rows_chunk(hkv, pages, kv_indices_len);
+  a.full_slots = (int)(kv_indices_len / a.chunk) + 1;
+  // Units of a row of four times the average length: the merge's groups are for these (more take another round).
+  const int64_t nu = rows > 1 ? 4 * ceil_div(ceil_div(pages, rows), a.chunk) : ceil_div(pages, a.chunk);
+  a.nsplit = (int)(nu < 2 ? 2 : (nu > 64 ? 64 : nu));
   a.part_ml = (float *)workspace;
-  a.part_acc = a.part_ml + (size_t)batch * hq * a.nsplit * 2;
+  a.part_acc = a.part_ml + (size_t)(a.full_slots + batch) * hq * 2;
   // Every row's units: its full ones (kv_indices_len / chunk in all) and its last one.
   const int units = (int)(kv_indices_len / a.chunk) + batch;
   if (dtype == DELTA_BF16)

@@ -56,8 +56,8 @@ int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const
                     const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices,
                     int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o, int64_t o_stride_t,
                     int64_t o_stride_h, float *lse, int batch, int hq, int hkv, int dtype, float sm_scale,
-                    void *workspace, hipStream_t stream, const char *who);
-size_t decode_rows_workspace_bytes(int batch, int hq, int hkv, int64_t pages);
+                    int rows, int64_t pages, void *workspace, hipStream_t stream, const char *who);
+size_t decode_rows_workspace_bytes(int batch, int hq, int64_t kv_indices_len);
 
 namespace {
 
@@ -634,13 +634,14 @@ int run_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h, const voi
   a.sm_scale = sm_scale;
   a.skip_single = rows;
   if (rows) {
-    const size_t need = decode_rows_workspace_bytes(batch, num_qo_heads, num_kv_heads, kv_indices_len);
+    const size_t need = decode_rows_workspace_bytes(batch, num_qo_heads, kv_indices_len);
     if (!workspace || workspace_bytes < need)
       return set_error(DELTA_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
     if ((uintptr_t)workspace & 255u) return set_error(DELTA_ERR_INVALID, "%s: workspace must be 256-byte aligned", who);
     const int rc = run_decode_rows(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
                                    kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
-                                   num_kv_heads, dtype, sm_scale, workspace, (hipStream_t)stream, who);
+                                   num_kv_heads, dtype, sm_scale, batch, kv_indices_len, workspace,
+                                   (hipStream_t)stream, who);
     if (rc || max_qo_len == 1) return rc;
   }
   if (dtype == DELTA_BF16)
@@ -668,7 +669,7 @@ extern "C" DELTA_EXPORT int delta_paged_prefill(const void *q, int64_t q_stride_
 extern "C" DELTA_EXPORT size_t delta_paged_prefill_rows_workspace_bytes(int batch, int num_qo_heads, int num_kv_heads,
                                                                         int64_t kv_indices_len) {
   if (batch <= 0 || num_qo_heads <= 0 || num_kv_heads <= 0 || kv_indices_len < 0) return 0;
-  return delta::decode_rows_workspace_bytes(batch, num_qo_heads, num_kv_heads, kv_indices_len);
+  return delta::decode_rows_workspace_bytes(batch, num_qo_heads, kv_indices_len);
 }
 
 extern "C" DELTA_EXPORT int delta_paged_prefill_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h,

@@ -93,6 +93,17 @@ def test_a_workspace_kept_for_long_rows_serves_shorter_ones(lib, batch, hq, hkv)
         assert max(need[:kept]) == need[kept - 1]
 
 
+def test_prefill_rows_workspace_is_bounded(lib):
+    """The partials of a prompt step's decoding rows: as many slots as the pages fill units, however they are
+    spread over the rows (one slot per row and unit of the longest row took 170 MB for 128 rows of 2000
+    pages), and never less for a step of fewer rows or pages."""
+    q = lib.delta_paged_prefill_rows_workspace_bytes
+    assert q(128, 40, 8, 128 * 2000) <= 25 << 20
+    assert q(32, 32, 8, 4063 + 31 * 6) <= 6 << 20
+    sizes = [[q(b, 32, 8, n) for n in (0, 1, 15, 16, 17, 1000, 16384, 16385, 100000, 1 << 20)] for b in (1, 8, 128)]
+    assert all(row == sorted(row) for row in sizes) and all(list(col) == sorted(col) for col in zip(*sizes))
+
+
 def test_small_attention_plans(lib):
     """Attention launches of 32-255 pairs: about 256 blocks, units of at most 128 pages.  Finer units were
     faster for full rows and slower for rows far below max_pages, which the plan cannot see.  (The query

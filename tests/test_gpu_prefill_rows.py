@@ -58,7 +58,7 @@ CASES = {
                          torch.float16),
     "one_row": ([(1, 5000)], 12, 2, torch.bfloat16),
     "all_single_g1": ([(1, 10 + 300 * i) for i in range(9)], 4, 4, torch.float16),
-    "long_row_past_the_unit_cap_g8": ([(1, 40000)] + [(1, 33)] * 300 + [(5, 5)], 8, 1, torch.bfloat16),
+    "long_row_beside_short_ones_g8": ([(1, 40000)] + [(1, 33)] * 300 + [(5, 5)], 8, 1, torch.bfloat16),
 }
 
 
