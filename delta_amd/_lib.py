@@ -12,7 +12,7 @@ LIB_PATH = Path(__file__).resolve().parent / "_delta_hip.so"
 
 DELTA_BF16 = 0
 DELTA_FP16 = 1
-ABI_VERSION = 202  # delta_abi_version() of the library these signatures describe
+ABI_VERSION = 203  # delta_abi_version() of the library these signatures describe
 
 _P = c_void_p
 
@@ -47,7 +47,7 @@ SIGNATURES = {
     "delta_paged_prefill_rows_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int64]),
     "delta_paged_prefill_rows": (c_int, [
         _P, c_int64, c_int64, _P, c_int64, _P, _P, _P, c_int64, _P, _P, c_int64, c_int64, _P,
-        c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, c_size_t, _P]),
+        c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int64, c_int, c_int64, c_int64, _P, c_size_t, _P]),
     "delta_paged_decode": (c_int, [
         _P, c_int64, c_int64,                 # q, strides
         _P, c_int64,                          # kv_cache, num_pages

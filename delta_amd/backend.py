@@ -49,9 +49,9 @@ class _StepCSR:
     """Page tables the attention ops read during one forward (prefill steps also carry the
     query-token CSR of the rows)."""
 
-    __slots__ = ("mode", "kv_indptr", "kv_indices", "kv_last", "max_pages", "qo_indptr", "max_qo")
+    __slots__ = ("mode", "kv_indptr", "kv_indices", "kv_last", "max_pages", "qo_indptr", "max_qo", "single_pages")
 
-    def __init__(self, mode, kv_indptr, kv_indices, kv_last, max_pages, qo_indptr=None, max_qo=1):
+    def __init__(self, mode, kv_indptr, kv_indices, kv_last, max_pages, qo_indptr=None, max_qo=1, single_pages=None):
         self.mode = mode
         self.kv_indptr = kv_indptr
         self.kv_indices = kv_indices
@@ -59,6 +59,7 @@ class _StepCSR:
         self.max_pages = max_pages
         self.qo_indptr = qo_indptr
         self.max_qo = max_qo
+        self.single_pages = single_pages  # pages of each prompt-step row of one new token
 
 
 class LMBackend:
@@ -254,7 +255,8 @@ class LMBackend:
                                     and K.paged_decode_scores_supported(B, hq, hkv, self.pages_per_slot, False))
         ws = max(K.decode_workspace_bytes(B, hq, hkv, self.pages_per_slot),
                  K.decode_workspace_bytes(B, hq, hkv, self.k_eff),
-                 K.paged_decode_scores_workspace_bytes(B, hkv, self.pages_per_slot), 256)
+                 K.paged_decode_scores_workspace_bytes(B, hkv, self.pages_per_slot),
+                 K.paged_prefill_workspace_bytes(B, hq, hkv, self.max_num_pages), 256)
         self.workspace = torch.empty(ws, dtype=torch.uint8, device=dev)
         self._pinned_tokens = torch.zeros(B, dtype=torch.long).pin_memory()
         with torch.device(dev):
@@ -360,7 +362,8 @@ class LMBackend:
         st = self._step
         if st.mode == "prefill":  # several query tokens per row: causal prefill kernel
             return self._profile_cuda_section("delta_prefill_attention", lambda: K.paged_prefill(
-                q, kv_cache, st.qo_indptr, st.kv_indptr, st.kv_indices, st.kv_last, max_qo_len=st.max_qo))
+                q, kv_cache, st.qo_indptr, st.kv_indptr, st.kv_indices, st.kv_last, max_qo_len=st.max_qo,
+                single_pages=st.single_pages, workspace=self.workspace))
         return self._profile_cuda_section("delta_full_attention", lambda: K.paged_decode(
             q, kv_cache, st.kv_indptr, st.kv_indices, st.kv_last, max_pages_per_row=st.max_pages,
             workspace=self.workspace, append=append))
@@ -849,7 +852,8 @@ class LMBackend:
         row_ind = torch.tensor(kv_indices, **i32)
         row_last = torch.tensor(rows_last, **i32)
         self._step = _StepCSR("prefill", row_ip, row_ind, row_last, max(len(p) for p in rows_pages),
-                              qo_indptr=qo_indptr, max_qo=max(qo_lens))
+                              qo_indptr=qo_indptr, max_qo=max(qo_lens),
+                              single_pages=[len(p) for n, p in zip(qo_lens, rows_pages) if n == 1])
         try:
             out = self.model(tokens, torch.tensor(offsets, **i32), qo_indptr, row_ind, row_ip, row_last)
         finally:

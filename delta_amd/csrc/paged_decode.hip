@@ -1558,13 +1558,13 @@ void launch_decode_rows(const DecodeArgs &a, int G, int units, hipStream_t strea
 }
 }  // namespace
 
-// Arguments as delta_paged_prefill, checked there; `rows` rows of one token hold `pages` pages (for the plan
-// only); workspace of decode_rows_workspace_bytes, 256-byte aligned.
+// Arguments as delta_paged_prefill, checked there; the rows of one token hold `pages` pages, the longest
+// `max_pages` (for the plan only); workspace of decode_rows_workspace_bytes, 256-byte aligned.
 int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache, int64_t num_pages,
                     const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices,
                     int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o, int64_t o_stride_t,
                     int64_t o_stride_h, float *lse, int batch, int hq, int hkv, int dtype, float sm_scale,
-                    int rows, int64_t pages, void *workspace, hipStream_t stream, const char *who) {
+                    int64_t pages, int64_t max_pages, void *workspace, hipStream_t stream, const char *who) {
   DecodeArgs a = {};
   a.q = (const uint16_t *)q;
   a.q_stride_b = q_stride_t;
@@ -1587,8 +1587,7 @@ int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const
   a.sm_scale = sm_scale;
   a.chunk = decode_rows_chunk(hkv, pages, kv_indices_len);
   a.full_slots = (int)(kv_indices_len / a.chunk) + 1;
-  // Units of a row of four times the average length: the merge's groups are for these (more take another round).
-  const int64_t nu = rows > 1 ? 4 * ceil_div(ceil_div(pages, rows), a.chunk) : ceil_div(pages, a.chunk);
+  const int64_t nu = ceil_div(max_pages, a.chunk);  // of the longest row, for the merge's groups (more take another round)
   a.nsplit = (int)(nu < 2 ? 2 : (nu > 64 ? 64 : nu));
   a.part_ml = (float *)workspace;
   a.part_acc = a.part_ml + (size_t)(a.full_slots + batch) * hq * 2;

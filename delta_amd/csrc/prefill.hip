@@ -56,7 +56,7 @@ int run_decode_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const
                     const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices,
                     int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o, int64_t o_stride_t,
                     int64_t o_stride_h, float *lse, int batch, int hq, int hkv, int dtype, float sm_scale,
-                    int rows, int64_t pages, void *workspace, hipStream_t stream, const char *who);
+                    int64_t pages, int64_t max_pages, void *workspace, hipStream_t stream, const char *who);
 size_t decode_rows_workspace_bytes(int batch, int hq, int64_t kv_indices_len);
 
 namespace {
@@ -97,6 +97,9 @@ struct PrefillArgs {
   int64_t o_stride_t, o_stride_h;
   float *lse;
   int batch, hq, hkv;
+  int64_t num_tokens;     // query tokens of all rows, -1: not known
+  int decode_rows;        // rows of one query token, their pages (for the choice of the blocks only)
+  int64_t decode_pages;
   int skip_single;  // rows of one query token are run_decode_rows'
   int row_tiles;    // the most tiles a row has (of max_qo_len tokens)
   int order;        // of the blocks: kBySlot, kByRow, kByTile
@@ -544,29 +547,40 @@ __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a
 // Whether blocks hold 8 waves instead of 4 (bt4 query tokens).  Where CUs would be left without a block, 4
 // waves spread a prompt over twice as many; where the chip is full anyway, 8 waves run a step faster (loads
 // two steps ahead, P.V of one wave under the softmax of the other).
-bool wide_blocks(int batch, int hkv, int bt4, int max_qo) {
+bool wide_blocks(const PrefillArgs &a, int bt4, int max_qo) {
   // The longest prompt alone is 850 4-wave blocks, nearly two rounds over the chip's 512.  us for 8 / 4
   // waves, 8 kv heads of 4 q heads: 3000 tokens (752 blocks) 88.9 / 86.0, 3200 (800) 94.1 / 93.3, 3500 (880)
   // 103.5 / 111, 4000 (1000) 131 / 142, 8192 (2048) 513 / 541; 2 kv heads of 6: 4096 (410) 105.5 / 94.6,
   // 6500 (650) 172 / 165, 8192 (820) 231.5 / 230, 16384 (1640) 833 / 849.
-  if (hkv * ceil_div(max_qo, bt4) >= 850) return true;
+  if (a.hkv * ceil_div(max_qo, bt4) >= 850) return true;
   // Prompts of one 8-wave block or two 4-wave ones, and the latter no longer fit one to a CU: 60 prompts
   // of 20, 4 kv heads of 7 (240 / 480 blocks) 10.2 / 12.6 us; 100 of 30, 2 of 6 (200 / 400) 10.9 / 11.8.
-  const int64_t blocks = (int64_t)batch * hkv;
-  return max_qo > bt4 && max_qo <= 2 * bt4 && blocks <= 256 && 2 * blocks > 256;
+  const int64_t blocks = (int64_t)a.batch * a.hkv;
+  if (max_qo > bt4 && max_qo <= 2 * bt4 && blocks <= 256 && 2 * blocks > 256) return true;
+  // Prompts continued over at least three times as many cached tokens, whose blocks all sweep about as far,
+  // and more 4-wave blocks than one to a CU: 1500 tokens at 16 k (376 blocks) 426 / 464 us, 2048 at 8 k (512)
+  // 284 / 298, 8 of 256 at 4 k (512) 139 / 149; but 1024 at 8 k (256) 222 / 195, 3000 at 8 k (2.7 times) 482 /
+  // 479, 2048 at 4 k (twice) 172 / 172.
+  if (a.num_tokens < 0) return false;
+  const int64_t tokens = a.num_tokens - a.decode_rows;
+  const int64_t cached = (a.kv_indices_len - a.decode_pages) * kPageSize - tokens;
+  return cached >= 3 * tokens && tokens * a.hkv >= 300 * (int64_t)bt4;
 }
 
 template <int DT, int G>
 void launch_prefill_g(PrefillArgs a, int max_qo, hipStream_t stream) {
-  const bool wide = wide_blocks(a.batch, a.hkv, 32 / G * 4, max_qo);
+  const bool wide = wide_blocks(a, 32 / G * 4, max_qo);
   const int bt = 32 / G * (wide ? 8 : 4);
   a.row_tiles = (int)ceil_div(max_qo, bt);
   const int64_t slots = (int64_t)a.batch * a.row_tiles;
   a.order = a.batch == 1 || slots * a.hkv <= (wide ? 256 : 512) ? kBySlot
             : a.batch <= kByTileRows && a.row_tiles <= 32 * 64  ? kByTile
                                                                 : kByRow;
-  const int64_t y = slots < 32768 ? slots : 32768;
-  const dim3 grid((unsigned)a.hkv, (unsigned)y, (unsigned)ceil_div(slots, y));
+  // Tiles of that many tokens over that many rows, at most: what is launched past the last one only exits, but
+  // a row of 5000 tokens beside 20 of 100 has 1540 slots too many (242 us, with the bound 215).
+  const int64_t most = a.num_tokens < 0 ? slots : (a.num_tokens + (int64_t)a.batch * (bt - 1)) / bt;
+  const int64_t used = a.order == kBySlot || slots < most ? slots : most, y = used < 32768 ? used : 32768;
+  const dim3 grid((unsigned)a.hkv, (unsigned)y, (unsigned)ceil_div(used, y));
   if (wide)
     hipLaunchKernelGGL((paged_prefill_kernel<DT, G, 8>), grid, dim3(512), 0, stream, a);
   else
@@ -587,17 +601,13 @@ void launch_prefill(const PrefillArgs &a, int G, int max_qo, hipStream_t stream)
   }
 }
 
-}  // namespace
-}  // namespace delta
-
-namespace delta {
-namespace {
-// rows: rows of one query token go to run_decode_rows (workspace of decode_rows_workspace_bytes).
+// With a workspace (of decode_rows_workspace_bytes) the rows of one query token go to run_decode_rows.
 int run_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache, int64_t num_pages,
                 const int32_t *qo_indptr, const int32_t *kv_indptr, const int32_t *kv_indices, int64_t kv_indices_len,
                 const int32_t *kv_last_page_len, void *o, int64_t o_stride_t, int64_t o_stride_h, float *lse, int batch,
-                int num_qo_heads, int num_kv_heads, int head_dim, int dtype, float sm_scale, int max_qo_len, bool rows,
-                void *workspace, size_t workspace_bytes, delta_stream_t stream, const char *who) {
+                int num_qo_heads, int num_kv_heads, int head_dim, int dtype, float sm_scale, int max_qo_len,
+                int64_t num_tokens, int decode_rows, int64_t decode_pages, int64_t decode_max_pages, void *workspace,
+                size_t workspace_bytes, delta_stream_t stream, const char *who) {
   clear_error();
   if (batch <= 0 || max_qo_len <= 0) return DELTA_OK;
   if (head_dim != kHeadDim) return set_error(DELTA_ERR_INVALID, "%s: head_dim must be 128", who);
@@ -632,16 +642,19 @@ int run_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h, const voi
   a.hq = num_qo_heads;
   a.hkv = num_kv_heads;
   a.sm_scale = sm_scale;
-  a.skip_single = rows;
-  if (rows) {
+  a.num_tokens = num_tokens;
+  a.decode_rows = decode_rows;
+  a.decode_pages = decode_pages;
+  a.skip_single = workspace != nullptr;
+  if (workspace) {
     const size_t need = decode_rows_workspace_bytes(batch, num_qo_heads, kv_indices_len);
-    if (!workspace || workspace_bytes < need)
+    if (workspace_bytes < need)
       return set_error(DELTA_ERR_WORKSPACE, "%s: workspace of %zu bytes needed, %zu given", who, need, workspace_bytes);
     if ((uintptr_t)workspace & 255u) return set_error(DELTA_ERR_INVALID, "%s: workspace must be 256-byte aligned", who);
     const int rc = run_decode_rows(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
                                    kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
-                                   num_kv_heads, dtype, sm_scale, batch, kv_indices_len, workspace,
-                                   (hipStream_t)stream, who);
+                                   num_kv_heads, dtype, sm_scale, decode_pages, decode_max_pages, workspace, (hipStream_t)stream,
+                                   who);
     if (rc || max_qo_len == 1) return rc;
   }
   if (dtype == DELTA_BF16)
@@ -662,7 +675,7 @@ extern "C" DELTA_EXPORT int delta_paged_prefill(const void *q, int64_t q_stride_
                                                 float sm_scale, int max_qo_len, delta_stream_t stream) {
   return delta::run_prefill(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
                             kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
-                            num_kv_heads, head_dim, dtype, sm_scale, max_qo_len, false, nullptr, 0, stream,
+                            num_kv_heads, head_dim, dtype, sm_scale, max_qo_len, -1, 0, 0, 0, nullptr, 0, stream,
                             "delta_paged_prefill");
 }
 
@@ -678,10 +691,19 @@ extern "C" DELTA_EXPORT int delta_paged_prefill_rows(const void *q, int64_t q_st
                                                      int64_t kv_indices_len, const int32_t *kv_last_page_len, void *o,
                                                      int64_t o_stride_t, int64_t o_stride_h, float *lse, int batch,
                                                      int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
-                                                     float sm_scale, int max_qo_len, void *workspace,
-                                                     size_t workspace_bytes, delta_stream_t stream) {
+                                                     float sm_scale, int max_qo_len, int64_t num_tokens,
+                                                     int decode_rows, int64_t decode_pages, int64_t decode_max_pages,
+                                                     void *workspace, size_t workspace_bytes,
+                                                     delta_stream_t stream) {
+  const char *who = "delta_paged_prefill_rows";
+  if (batch > 0 && max_qo_len > 0 &&
+      (num_tokens < 0 || decode_rows < 0 || decode_rows > batch || decode_pages < 0 || decode_pages > kv_indices_len ||
+       decode_max_pages < 0 || decode_max_pages > decode_pages)) {
+    delta::clear_error();
+    return delta::set_error(DELTA_ERR_INVALID, "%s: num_tokens, decode_rows, decode_pages or decode_max_pages out of range", who);
+  }
   return delta::run_prefill(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
                             kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
-                            num_kv_heads, head_dim, dtype, sm_scale, max_qo_len, true, workspace, workspace_bytes, stream,
-                            "delta_paged_prefill_rows");
+                            num_kv_heads, head_dim, dtype, sm_scale, max_qo_len, num_tokens, decode_rows, decode_pages,
+                            decode_max_pages, workspace, workspace_bytes, stream, who);
 }

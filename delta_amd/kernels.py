@@ -10,7 +10,7 @@ from __future__ import annotations
 import ctypes
 import math
 from dataclasses import dataclass
-from typing import Optional
+from typing import Optional, Sequence
 
 import torch
 
@@ -273,14 +273,29 @@ def paged_decode_scores(q: torch.Tensor, kv_cache: torch.Tensor, kv_indptr: torc
     return out, scores
 
 
+def _split_decode_rows(max_qo_len: int, tokens: int, hq: int, hkv: int, pages: int, longest: int) -> bool:
+    """Whether a prompt step's rows of one new token (``pages`` pages, the longest ``longest``) go to split
+    decode units.  One prefill block per kv head sweeps such a row alone, 0.33 us a page; the rows launch and
+    its merge cost ~11 us (5 without prompts), in front of the prompts, and the rows' bytes.  So the longest
+    row has to outlast the longest prompt (0.022 us a token) by that, or, where the prompts alone are more
+    blocks than the chip holds and the row starts behind them, to be worth it by itself; and where rows times kv
+    heads keep the CUs streaming anyway there is less to gain (us without / with, 8 kv heads of 4 q heads: one row
+    of 63 / 126 pages beside 50 tokens 24 / 19, 44 / 20, beside 1000 29 / 41, 47 / 43, beside 2000 55 / 68, 57 /
+    68; of 82 / 188 beside 4000 151 / 151, 180 / 152; 30 rows of 126 / 188 beside 300 55 / 63, 79 / 85, 31 of
+    64-500 beside 777 180 / 138)."""
+    if max_qo_len == 1:
+        least = 24.0
+    elif tokens * hkv > 512 * 4 * (32 // (hq // hkv)):
+        least = 90.0
+    else:
+        least = 40.0 + 0.065 * max_qo_len
+    return longest > least + min(0.0033 * hkv * pages, 160.0)
+
+
 def _prefill_has_decode_rows(tokens: int, batch: int, max_qo_len: int, pages: int) -> bool:
-    """Whether a prompt step is likely to hold rows with one new token and a long cache: the rows but
-    the longest average under half its tokens (the row lengths themselves are on the device), and hold
-    1024 cached tokens or more on average (1344 below 16 rows).  One prefill block per kv head sweeps
-    such a row alone (31 rows of 1-8 k tokens beside a 777-token prompt: 207 us against 147 with split
-    decode units; 30 of 0.5-2.7 k beside 8 short prompts: 67 / 44; 5 of 0.5-2 k beside 100 tokens: 46 / 32),
-    but the two extra launches cost ~5 us: 5 rows of 0.5-1 k 28-30 / 33, 30 of them 45.8 / 46.5, 5 of
-    0.5-1.4 k beside prompts at 1000 tokens 44-46 / 48."""
+    """Whether a prompt step whose caller does not say so is likely to hold rows with one new token and a
+    long cache: the rows but the longest average under half its tokens (the row lengths themselves are on the
+    device), and hold 1024 cached tokens or more on average (1344 below 16 rows)."""
     if batch <= 0 or max_qo_len <= 0:
         return False
     long_pages = 64 if batch >= 16 else 84
@@ -290,12 +305,23 @@ def _prefill_has_decode_rows(tokens: int, batch: int, max_qo_len: int, pages: in
             and pages - (max_qo_len + 15) // 16 >= long_pages * (batch - 1))
 
 
+def paged_prefill_workspace_bytes(batch: int, hq: int, hkv: int, pages: int) -> int:
+    """Bytes of ``paged_prefill``'s workspace for steps of up to ``batch`` rows and ``pages`` pages."""
+    return int(_lib.query("delta_paged_prefill_rows_workspace_bytes", batch, hq, hkv, pages))
+
+
 def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, qo_indptr: torch.Tensor,
                   kv_indptr: torch.Tensor, kv_indices: torch.Tensor, kv_last_page_len: torch.Tensor, *,
                   max_qo_len: int, sm_scale: Optional[float] = None, out: Optional[torch.Tensor] = None,
-                  lse: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """Causal paged prefill attention (``delta_paged_prefill``); q/out [nnz, Hq, 128]."""
-    dev = _check_cuda(q, kv_cache, qo_indptr, kv_indptr, kv_indices, kv_last_page_len, out, lse)
+                  lse: Optional[torch.Tensor] = None, single_pages: Optional[Sequence[int]] = None,
+                  workspace: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """Causal paged prefill attention (``delta_paged_prefill_rows``); q/out [nnz, Hq, 128].
+
+    ``single_pages``: the pages of each row of exactly one new token, where the caller knows them (they
+    choose how those rows run, no result depends on them); without it they are guessed from the totals.
+    ``workspace`` (``paged_prefill_workspace_bytes``) holds those rows' partials; without one they are
+    allocated for the call, and where that fails the step runs without them."""
+    dev = _check_cuda(q, kv_cache, qo_indptr, kv_indptr, kv_indices, kv_last_page_len, out, lse, workspace)
     _check_cache(kv_cache)
     hq, hkv = _check_heads(q, kv_cache)
     B = qo_indptr.numel() - 1
@@ -312,16 +338,33 @@ def paged_prefill(q: torch.Tensor, kv_cache: torch.Tensor, qo_indptr: torch.Tens
         raise ValueError("lse must be contiguous fp32 [nnz, Hq]")
     if sm_scale is None:
         sm_scale = 1.0 / math.sqrt(HEAD_DIM)
-    args = (q.data_ptr(), q.stride(0), q.stride(1), kv_cache.data_ptr(), kv_cache.shape[0], qo_indptr.data_ptr(),
-            kv_indptr.data_ptr(), kv_indices.data_ptr(), kv_indices.numel(), kv_last_page_len.data_ptr(),
-            out.data_ptr(), out.stride(0), out.stride(1), _ptr(lse), int(B), hq, hkv, HEAD_DIM, _dtype_code(q),
-            float(sm_scale), int(max_qo_len))
-    if _prefill_has_decode_rows(q.shape[0], B, int(max_qo_len), kv_indices.numel()):
-        nbytes = int(_lib.query("delta_paged_prefill_rows_workspace_bytes", B, hq, hkv, kv_indices.numel()))
-        ws = torch.empty(nbytes, dtype=torch.uint8, device=dev)  # of this call: safe on any stream, in any capture
-        _lib.call("delta_paged_prefill_rows", *args, ws.data_ptr(), nbytes, _stream(dev))
+    pages = kv_indices.numel()
+    if single_pages is not None:
+        rows, total, longest = len(single_pages), sum(single_pages), max(single_pages, default=0)
+        if rows > B or total > pages or min(single_pages, default=0) < 0:
+            raise ValueError(f"single_pages names {rows} rows of {total} pages, the step has {B} of {pages}")
+        split = _split_decode_rows(int(max_qo_len), q.shape[0], hq, hkv, total, longest)
     else:
-        _lib.call("delta_paged_prefill", *args, _stream(dev))
+        split = _prefill_has_decode_rows(q.shape[0], B, int(max_qo_len), pages)
+        rows = total = longest = 0
+        if split:
+            rows = B if max_qo_len == 1 else B - 1
+            total = pages if max_qo_len == 1 else pages - (int(max_qo_len) + 15) // 16
+            longest = min(total, 4 * -(-total // rows))
+    if split:
+        need = paged_prefill_workspace_bytes(B, hq, hkv, pages)
+        if workspace is None:
+            try:  # of this call: safe on any stream, in any capture
+                workspace = torch.empty(need, dtype=torch.uint8, device=dev)
+            except torch.OutOfMemoryError:
+                split = False
+        elif workspace.numel() * workspace.element_size() < need:
+            raise ValueError(f"workspace too small: {need} bytes needed")
+    _lib.call("delta_paged_prefill_rows", q.data_ptr(), q.stride(0), q.stride(1), kv_cache.data_ptr(), kv_cache.shape[0],
+              qo_indptr.data_ptr(), kv_indptr.data_ptr(), kv_indices.data_ptr(), pages, kv_last_page_len.data_ptr(),
+              out.data_ptr(), out.stride(0), out.stride(1), _ptr(lse), int(B), hq, hkv, HEAD_DIM, _dtype_code(q),
+              float(sm_scale), int(max_qo_len), q.shape[0], rows, total, longest, workspace.data_ptr() if split else None,
+              workspace.numel() * workspace.element_size() if split else 0, _stream(dev))
     return out
 
 

@@ -213,10 +213,14 @@ int delta_paged_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h,
                         int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
                         float sm_scale, int max_qo_len, delta_stream_t stream);
 
-/* delta_paged_prefill for steps in which prompts join rows that are decoding: the same o and lse, with
- * the rows of exactly one query token attended by split decode units (a merge launch follows) instead of
- * one prefill block per kv head each.  workspace: delta_paged_prefill_rows_workspace_bytes bytes, 256-byte
- * aligned. */
+/* delta_paged_prefill with what the caller knows of the step; the same o and lse.
+ *   num_tokens        query tokens of all rows (>= qo_indptr[batch]): it bounds the grid
+ *   decode_rows       rows of exactly one query token, decode_pages their pages in total, decode_max_pages
+ *                     those of the longest one (for the launch plan: no result depends on them)
+ *   workspace         NULL, or delta_paged_prefill_rows_workspace_bytes bytes, 256-byte aligned: the rows
+ *                     of exactly one query token are then attended by split decode units (a merge launch
+ *                     follows) instead of one prefill block per kv head each.  The bytes never decrease
+ *                     with batch or kv_indices_len, so one sized for the largest step serves all. */
 size_t delta_paged_prefill_rows_workspace_bytes(int batch, int num_qo_heads, int num_kv_heads,
                                                 int64_t kv_indices_len);
 int delta_paged_prefill_rows(const void *q, int64_t q_stride_t, int64_t q_stride_h, const void *kv_cache,
@@ -224,9 +228,9 @@ int delta_paged_prefill_rows(const void *q, int64_t q_stride_t, int64_t q_stride
                              const int32_t *kv_indices, int64_t kv_indices_len,
                              const int32_t *kv_last_page_len, void *o, int64_t o_stride_t, int64_t o_stride_h,
                              float *lse, int batch, int num_qo_heads, int num_kv_heads, int head_dim, int dtype,
-                             float sm_scale, int max_qo_len, void *workspace, size_t workspace_bytes,
-                             delta_stream_t stream);
-
+                             float sm_scale, int max_qo_len, int64_t num_tokens, int decode_rows,
+                             int64_t decode_pages, int64_t decode_max_pages, void *workspace,
+                             size_t workspace_bytes, delta_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Page scoring (del3_legacy_softmax)                                         */

@@ -33,7 +33,7 @@ def build(rows, hq, hkv, dtype, seed, spoil=True):
                 last=torch.tensor([n % 16 for _, n in rows], **i32))
 
 
-def launch(c, rows, max_qo, scale=128 ** -0.5):
+def launch(c, rows, max_qo, scale=128 ** -0.5, hints=None):
     q, kv = c["q"], c["kv"]
     hq, hkv, B = q.shape[1], kv.shape[3], c["qo"].numel() - 1
     o = torch.full_like(q, 7.0)
@@ -45,7 +45,9 @@ def launch(c, rows, max_qo, scale=128 ** -0.5):
     if rows:
         n = _lib.query("delta_paged_prefill_rows_workspace_bytes", B, hq, hkv, c["ids"].numel())
         ws = torch.full((n,), 255, dtype=torch.uint8, device=DEV)  # NaN partials where none are written
-        _lib.call("delta_paged_prefill_rows", *args, ws.data_ptr(), n, stream)
+        pages = c["ids"].numel()
+        hints = (B, pages, pages) if hints is None else hints
+        _lib.call("delta_paged_prefill_rows", *args, q.shape[0], *hints, ws.data_ptr(), n, stream)
     else:
         _lib.call("delta_paged_prefill", *args, stream)
     torch.cuda.synchronize()
@@ -144,7 +146,8 @@ def test_paged_prefill_takes_the_rows_path_where_it_should():
     args = (c["q"], c["kv"], c["qo"], c["ptr"], c["ids"], c["last"])
     assert K._prefill_has_decode_rows(c["q"].shape[0], len(rows), 40, c["ids"].numel())
     o = K.paged_prefill(*args, max_qo_len=40)
-    assert torch.equal(o, launch(c, True, 40)[0])
+    total = c["ids"].numel() - 3  # the guess: all rows but the longest prompt
+    assert torch.equal(o, launch(c, True, 40, hints=(7, total, min(total, 4 * -(-total // 7))))[0])
     g = torch.cuda.CUDAGraph()
     with torch.cuda.graph(g):
         og = K.paged_prefill(*args, max_qo_len=40)
@@ -153,3 +156,69 @@ def test_paged_prefill_takes_the_rows_path_where_it_should():
         g.replay()
         torch.cuda.synchronize()
         assert torch.equal(og, o)
+
+
+def test_paged_prefill_takes_the_callers_word_for_the_decoding_rows(monkeypatch):
+    """With ``single_pages`` nothing is guessed: prompts alone get no split launch, one long decoding row
+    beside longer prompts does, on the caller's workspace and without an allocation; what does not fit in
+    memory is not needed."""
+    sent = []
+    real = _lib.call
+    monkeypatch.setattr(_lib, "call", lambda name, *a: (sent.append((name, a)), real(name, *a))[1])
+    gave_workspace = lambda: sent[-1][1][-3]
+    prompts = build([(400, 400), (150, 150)], 8, 2, torch.bfloat16, seed=1)
+    joined = build([(300, 300), (290, 290), (1, 6000), (1, 20)], 8, 2, torch.bfloat16, seed=2)
+    singles = [6000 // 16 + 1, 20 // 16 + 1]
+    call = lambda c, mx, **kw: K.paged_prefill(c["q"], c["kv"], c["qo"], c["ptr"], c["ids"], c["last"], max_qo_len=mx, **kw)
+
+    o = call(prompts, 400, single_pages=[])
+    assert gave_workspace() is None and torch.equal(o, launch(prompts, False, 400)[0])
+    plain, split = launch(joined, False, 300)[0], launch(joined, True, 300, hints=(2, sum(singles), singles[0]))[0]
+    assert not torch.equal(plain, split)
+    ws = torch.empty(K.paged_prefill_workspace_bytes(4, 8, 2, joined["ids"].numel()), dtype=torch.uint8, device=DEV)
+    out = torch.empty_like(joined["q"])
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_stats()["allocation.all.allocated"]
+    call(joined, 300, single_pages=singles, workspace=ws, out=out)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+    assert gave_workspace() == ws.data_ptr() and torch.equal(out, split)
+    assert torch.equal(call(joined, 300, single_pages=singles), split)
+    with pytest.raises(ValueError, match="workspace too small"):
+        call(joined, 300, single_pages=singles, workspace=ws[:1024])
+    with pytest.raises(ValueError, match="single_pages names"):
+        call(joined, 300, single_pages=[10 ** 6])
+
+    def full(*a, **kw):
+        if kw.get("dtype") is torch.uint8:
+            raise torch.OutOfMemoryError("no room")
+        return empty(*a, **kw)
+
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", full)
+    assert torch.equal(call(joined, 300, single_pages=singles), plain)
+    assert gave_workspace() is None
+
+
+def test_engine_names_the_decoding_rows_of_its_prompt_steps(monkeypatch):
+    """Requests that join a running one: each prompt step passes the pages of the rows that decode and the
+    engine's own workspace, which is large enough for a step over the whole pool."""
+    from delta_amd.backend import LMBackend
+    be = LMBackend(dtype=torch.bfloat16, device=DEV, cuda_graph_decode=True)
+    be.is_main_process = False
+    be.load_model("random:tiny-test", n_layer=2, seed=1)
+    be.setup_caches(max_batch_size=2, max_seq_length=400)
+    seen = []
+    real = K.paged_prefill
+    monkeypatch.setattr(K, "paged_prefill", lambda q, kv, qo, *a, **kw: (seen.append((qo.tolist(), a, kw)),
+                                                                        real(q, kv, qo, *a, **kw))[1])
+    be.add_requests([torch.arange(1, n) for n in (90, 30, 55)], [200, 36, 70], [])
+    be.run_scheduler_loop()
+    joins = 0
+    for qo, (ptr, ids, last), kw in seen:
+        n = [b - a for a, b in zip(qo, qo[1:])]
+        pages = [b - a for a, b in zip(ptr.tolist(), ptr.tolist()[1:])]
+        assert kw["single_pages"] == [p for p, m in zip(pages, n) if m == 1]
+        assert kw["workspace"] is be.workspace
+        joins += bool(kw["single_pages"])
+    assert joins
+    assert be.workspace.numel() >= K.paged_prefill_workspace_bytes(2, 4, 2, be.max_num_pages)

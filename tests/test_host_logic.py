@@ -247,3 +247,15 @@ def test_qkv_bias_and_row_major_gate_up_merge_on_load():
         assert torch.equal(a.attention.wqkv.weight, b.attention.wqkv.weight)
         assert torch.equal(a.attention.wqkv.bias, b.attention.wqkv.bias)
         assert torch.equal(a.feed_forward.w13_t.t(), b.feed_forward.w13)
+
+
+@pytest.mark.parametrize("max_qo,tokens,hq,hkv,singles,split", [
+    (4096, 5596, 32, 8, [], False),                    # two prompts, no decoding row
+    (4000, 8001, 32, 8, [1001], True),                 # one long row beside two long prompts
+    (777, 808, 32, 8, [64 + 14 * i for i in range(31)], True),
+    (400, 415, 32, 8, [38] * 15, False),               # short rows: over before the extra launches are
+    (2000, 2001, 12, 2, [100], False), (2000, 2001, 12, 2, [200], True),
+    (1, 5, 28, 4, [20] * 5, False), (1, 5, 28, 4, [60] * 5, True)])
+def test_prompt_step_splits_the_decoding_rows_that_outlast_it(max_qo, tokens, hq, hkv, singles, split):
+    from delta_amd import kernels as K
+    assert K._split_decode_rows(max_qo, tokens, hq, hkv, sum(singles), max(singles, default=0)) is split
