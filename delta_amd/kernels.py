@@ -295,14 +295,16 @@ def _split_decode_rows(max_qo_len: int, tokens: int, hq: int, hkv: int, pages: i
 def _prefill_has_decode_rows(tokens: int, batch: int, max_qo_len: int, pages: int) -> bool:
     """Whether a prompt step whose caller does not say so is likely to hold rows with one new token and a
     long cache: the rows but the longest average under half its tokens (the row lengths themselves are on the
-    device), and hold 1024 cached tokens or more on average (1344 below 16 rows)."""
+    device), hold 1024 cached tokens or more on average (1344 below 16 rows), and four times their new tokens
+    (prompts without a past hold their new ones: 4096 and 1500 tokens, 162 us and 4 for two idle launches)."""
     if batch <= 0 or max_qo_len <= 0:
         return False
     long_pages = 64 if batch >= 16 else 84
     if max_qo_len == 1:
         return pages >= long_pages * batch
-    return (batch > 1 and 2 * (tokens - max_qo_len) < (batch - 1) * max_qo_len
-            and pages - (max_qo_len + 15) // 16 >= long_pages * (batch - 1))
+    rest, rest_pages = tokens - max_qo_len, pages - (max_qo_len + 15) // 16
+    return (batch > 1 and 2 * rest < (batch - 1) * max_qo_len and rest_pages >= long_pages * (batch - 1)
+            and PAGE_SIZE * rest_pages >= 4 * rest)
 
 
 def paged_prefill_workspace_bytes(batch: int, hq: int, hkv: int, pages: int) -> int:

@@ -259,3 +259,10 @@ def test_qkv_bias_and_row_major_gate_up_merge_on_load():
 def test_prompt_step_splits_the_decoding_rows_that_outlast_it(max_qo, tokens, hq, hkv, singles, split):
     from delta_amd import kernels as K
     assert K._split_decode_rows(max_qo, tokens, hq, hkv, sum(singles), max(singles, default=0)) is split
+
+
+def test_prompts_without_a_past_are_not_guessed_to_be_decoding_rows():
+    from delta_amd import kernels as K
+    assert not K._prefill_has_decode_rows(4096 + 1500, 2, 4096, 257 + 94)
+    assert not K._prefill_has_decode_rows(8000 + 2000, 2, 8000, 501 + 126)
+    assert K._prefill_has_decode_rows(4096 + 1, 2, 4096, 257 + 94)
