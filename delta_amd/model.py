@@ -218,10 +218,8 @@ def dense(x: Tensor, layer: nn.Linear) -> Tensor:
         rows = x.numel() // x.shape[-1]
         if rows <= _SKINNY_ROWS_ANY or w.numel() * w.element_size() <= _SKINNY_MAX_WEIGHT_BYTES:
             return K.gemm_skinny(x, w, layer.bias)
-    elif w.shape[0] >= _ROWS128_WIDE and w.shape[1] <= 2048 and K.gemm_rows128_ok(x, w):
-        rows = x.numel() // x.shape[-1]
-        if _ROWS32_MAX < rows <= 64 and K.gemm_rows128_splits(rows, *w.shape) == 1:
-            return K.gemm_rows128(x, w, layer.bias)
+    elif _rows128_head(x.numel() // max(x.shape[-1], 1), *w.shape) and K.gemm_rows128_ok(x, w):
+        return K.gemm_rows128(x, w, layer.bias)
     return layer(x)
 
 
@@ -238,12 +236,18 @@ _ROWS32_MAX = 32
 # 32.1, w1|w3 65-73 vs 73 and 5).  It stays on hipBLASLt where that is faster: past 64 rows weights of
 # fewer than 8 M elements (the 1.5B wo: 8.5 vs 7.1, and the norm's partials come on top) and gate/up
 # launches of more than 256 blocks of 64 columns, a second pass over the CUs (Qwen2.5-7B w1|w3: 80-89
-# vs 72); wqkv and lm_head too, whose consumers sum no partials (14B wqkv unsplit 40 vs 33), but for
-# an lm_head of few features at up to 64 rows (1.5B, K = 1536: 100 vs 113; 8B, K = 4096: 212 vs 211).
+# vs 72); wqkv and most lm_heads too, whose consumers sum no partials (see _rows128_head).
 _ROWS128_MAX = 128
-_ROWS128_WIDE = 32768
 _ROWS128_MIN_WEIGHT = 8 << 20
 _ROWS128_GLU_MAX = 64 * 256
+
+
+def _rows128_head(rows: int, N: int, Kd: int) -> bool:
+    """A wide lm_head of few features, unsplit (wqkv and other lm_heads stay on hipBLASLt: 14B wqkv unsplit 40 vs 33
+    us, 8B lm_head of 4096 features 212 vs 211).  940 blocks of 128 columns are nearly four passes over the CUs, so
+    the last one matters little: 0.52-1.03 of hipBLASLt for 120064-256000 columns and 1024-2048 features;
+    32768 and 50304 columns 1.0-1.36, 512 features up to 1.33."""
+    return _ROWS32_MAX < rows <= 64 and N >= 120000 and 1024 <= Kd <= 2048 and K.gemm_rows128_splits(rows, N, Kd) == 1
 
 
 def dense_to_norm(x: Tensor, layer: nn.Linear):

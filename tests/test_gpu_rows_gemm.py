@@ -2,7 +2,7 @@
 import pytest
 import torch
 
-from delta_amd import _lib, kernels as K
+from delta_amd import _lib, kernels as K, model
 from delta_amd.model import FeedForward, ModelArgs
 
 pytestmark = pytest.mark.gpu
@@ -19,6 +19,7 @@ DEV = "cuda:0"
     (128, 5120, 4160, True),    # 192-column blocks, N past a whole number of them, 65 k steps
     (100, 16400, 320, True),    # unsplit, rows and columns ragged
     (1, 208, 192, False),
+    (64, 33296, 1536, False),   # unsplit, 24 k steps (four x slabs), columns past a whole number of blocks
 ])
 def test_gemm_rows128_matches_fp32_reference(dtype, M, N, Kd, bias):
     """Partials sum to the product (fp32 sums of Kd products: 1e-5 of the sum of magnitudes, as for
@@ -85,6 +86,24 @@ def test_ffn_at_33_to_128_rows_matches_the_library_path():
                 y = (y.sum(0) if y.dtype == torch.float32 else y.float()).view(rows, 512)
                 # both round silu(g) * u and the output to bf16: a few ulps of the row's magnitude
                 assert (y - ref).abs().max().item() <= 4 * 2 ** -8 * ref.abs().max().item()
+
+
+@torch.inference_mode()
+@pytest.mark.parametrize("N,Kd,rows", [(120016, 1024, (32, 33, 64, 65)), (32768, 2048, (33, 64))])
+def test_lm_head_on_the_kernel_only_where_it_is_wide(N, Kd, rows, monkeypatch):
+    """dense() on either side of the lm_head rule against fp32 products rounded once."""
+    ran = []
+    gemm = K.gemm_rows128
+    monkeypatch.setattr(K, "gemm_rows128", lambda x, *a: (ran.append(x.shape[1]), gemm(x, *a))[1])
+    gen = torch.Generator(device=DEV).manual_seed(N)
+    layer = torch.nn.Linear(Kd, N, bias=False, device=DEV, dtype=torch.bfloat16)
+    layer.weight.normal_(0, 0.05, generator=gen)
+    for m in rows:
+        x = torch.randn(1, m, Kd, generator=gen, device=DEV).bfloat16()
+        y = model.dense(x, layer)[0].float()
+        ref, mag = x[0].float() @ layer.weight.float().T, x[0].float().abs() @ layer.weight.float().abs().T
+        assert torch.all((y - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5 * mag + 1e-6)
+    assert ran == ([33, 64] if N >= 120000 else [])
 
 
 def test_gemm_rows128_errors():

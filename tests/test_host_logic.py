@@ -266,3 +266,11 @@ def test_prompts_without_a_past_are_not_guessed_to_be_decoding_rows():
     assert not K._prefill_has_decode_rows(4096 + 1500, 2, 4096, 257 + 94)
     assert not K._prefill_has_decode_rows(8000 + 2000, 2, 8000, 501 + 126)
     assert K._prefill_has_decode_rows(4096 + 1, 2, 4096, 257 + 94)
+
+
+def test_lm_head_kernel_only_for_wide_heads():
+    from delta_amd.model import _rows128_head
+    assert _rows128_head(64, 151936, 1536) and _rows128_head(33, 128256, 2048)
+    for rows, n, k in ((64, 32768, 2048), (64, 50304, 1024), (64, 128256, 512), (64, 128256, 4096),
+                       (32, 151936, 1536), (65, 151936, 1536)):
+        assert not _rows128_head(rows, n, k)
