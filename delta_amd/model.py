@@ -233,13 +233,21 @@ _ROWS32_MAX = 32
 # At 33-128 token rows the same projections, and the merged w1|w3 with SiLU-mul, go to
 # delta_gemm_rows128 (us, against hipBLASLt; 64 rows: DeepSeek-R1-Distill-Qwen-1.5B w2 9.8 vs 25.4, wo
 # 4.9 vs 7.5, w1|w3 18.2 vs 18.7 and a 5 us SiLU-mul; 128 rows: Qwen2.5-14B w2 34.9 vs 73.9, wo 18.9 vs
-# 32.1, w1|w3 65-73 vs 73 and 5).  It stays on hipBLASLt where that is faster: past 64 rows weights of
-# fewer than 8 M elements (the 1.5B wo: 8.5 vs 7.1, and the norm's partials come on top) and gate/up
-# launches of more than 256 blocks of 64 columns, a second pass over the CUs (Qwen2.5-7B w1|w3: 80-89
+# 32.1, w1|w3 65-73 vs 73 and 5).  It stays on hipBLASLt where that is faster: past 64 rows most square
+# weights (see _rows128_to_norm) and gate/up launches of more than 256 blocks of 64 columns, a second pass over the CUs (Qwen2.5-7B w1|w3: 80-89
 # vs 72); wqkv and most lm_heads too, whose consumers sum no partials (see _rows128_head).
 _ROWS128_MAX = 128
-_ROWS128_MIN_WEIGHT = 8 << 20
 _ROWS128_GLU_MAX = 64 * 256
+
+
+def _rows128_to_norm(rows: int, N: int, Kd: int) -> bool:
+    """A projection whose consumer sums its partials (the times include that norm).  33-64 rows: every shape
+    tried (0.34-1.02 of hipBLASLt and the norm).  65-128: long K, whose splits fill the chip (1536 x 8960
+    0.87-0.96, 4096 x 14336 0.46-0.7; 1024 x 8192 1.0-1.12), or from 24 M elements on (5120 x 5120 0.75-1.02;
+    4096 x 4096 1.01-1.10 but for 96 and 128 rows, 3584 x 3584 1.0-1.2, 1536 x 1536 1.04-1.26)."""
+    if rows <= 64:
+        return rows > _ROWS32_MAX
+    return rows <= _ROWS128_MAX and (N * Kd >= 24 << 20 or (Kd >= 8192 and N * Kd >= 12 << 20))
 
 
 def _rows128_head(rows: int, N: int, Kd: int) -> bool:
@@ -258,8 +266,7 @@ def dense_to_norm(x: Tensor, layer: nn.Linear):
     if rows > _SKINNY_ROWS_ANY and rows <= _ROWS32_MAX and K.gemm_skinny_ok(x, w) and w.shape[0] % 64 == 0:
         r = K.gemm_rows32(x, w, layer.bias)
         return r if r.dtype == torch.float32 else r.view(*x.shape[:-1], w.shape[0])
-    if _ROWS32_MAX < rows <= _ROWS128_MAX and K.gemm_rows128_ok(x, w) \
-            and (rows <= 64 or w.numel() >= _ROWS128_MIN_WEIGHT):
+    if _rows128_to_norm(rows, *w.shape) and K.gemm_rows128_ok(x, w):
         r = K.gemm_rows128(x, w, layer.bias)
         return r if r.dtype == torch.float32 else r.view(*x.shape[:-1], w.shape[0])
     return dense(x, layer)

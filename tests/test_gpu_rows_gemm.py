@@ -106,6 +106,25 @@ def test_lm_head_on_the_kernel_only_where_it_is_wide(N, Kd, rows, monkeypatch):
     assert ran == ([33, 64] if N >= 120000 else [])
 
 
+@torch.inference_mode()
+@pytest.mark.parametrize("N,Kd,partial_rows", [(1536, 8960, (33, 64, 65, 128)), (4096, 4096, (33, 64)), (5120, 5120, (33, 64, 65, 128))])
+def test_dense_to_norm_form_and_values(N, Kd, partial_rows):
+    """Rows either side of 32, 64 and 128: fp32 partials where the kernel runs (here all split), else the rounded
+    output; both the fp32 products."""
+    gen = torch.Generator(device=DEV).manual_seed(Kd)
+    layer = torch.nn.Linear(Kd, N, bias=False, device=DEV, dtype=torch.bfloat16)
+    layer.weight.normal_(0, 0.02, generator=gen)
+    for m in (33, 64, 65, 128, 129):
+        x = torch.randn(1, m, Kd, generator=gen, device=DEV).bfloat16()
+        y = model.dense_to_norm(x, layer)
+        ref, mag = x[0].float() @ layer.weight.float().T, x[0].float().abs() @ layer.weight.float().abs().T
+        if m in partial_rows:
+            assert y.dtype == torch.float32 and torch.all((y.sum(0) - ref).abs() <= 1e-5 * mag + 1e-6)
+        else:
+            assert y.dtype == torch.bfloat16 and tuple(y.shape) == (1, m, N)
+            assert torch.all((y[0].float() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5 * mag + 1e-6)
+
+
 def test_gemm_rows128_errors():
     x = torch.zeros(33, 64, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)

@@ -268,9 +268,23 @@ def test_prompts_without_a_past_are_not_guessed_to_be_decoding_rows():
     assert K._prefill_has_decode_rows(4096 + 1, 2, 4096, 257 + 94)
 
 
+TABLE = {"llama-3-8b": (14336, 4096), "Qwen2.5-7b": (18944, 3584), "Qwen2.5-14b": (13824, 5120),
+         "DeepSeek-R1-Distill-Qwen-1.5B": (8960, 1536)}
+
+
 def test_lm_head_kernel_only_for_wide_heads():
     from delta_amd.model import _rows128_head
     assert _rows128_head(64, 151936, 1536) and _rows128_head(33, 128256, 2048)
     for rows, n, k in ((64, 32768, 2048), (64, 50304, 1024), (64, 128256, 512), (64, 128256, 4096),
                        (32, 151936, 1536), (65, 151936, 1536)):
         assert not _rows128_head(rows, n, k)
+
+
+def test_norm_projection_kernel_past_64_rows_needs_long_k_or_a_large_weight():
+    from delta_amd.model import _rows128_to_norm
+    for inter, dim in TABLE.values():  # w2
+        assert all(_rows128_to_norm(r, dim, inter) for r in (33, 64, 65, 128))
+    for dim in (1536, 3584, 4096):  # wo
+        assert _rows128_to_norm(64, dim, dim) and not _rows128_to_norm(65, dim, dim)
+    assert _rows128_to_norm(65, 5120, 5120) and not _rows128_to_norm(96, 1024, 8192)
+    assert not _rows128_to_norm(32, 4096, 14336) and not _rows128_to_norm(129, 4096, 14336)
