@@ -198,7 +198,7 @@ class LMBackend:
         dev = self.device
         self.max_length = max_seq_length
         self.batch_size = max_batch_size
-        if max_batch_size <= model_mod._ROWS128_MAX:
+        if model_mod.row_major_gate_up(max_batch_size, cfg.intermediate_size, cfg.dim):
             # the gate|up GEMM of this engine's decode steps runs on delta_gemm_skinny (<= 8 rows),
             # delta_gemm_rows32_silu or delta_gemm_rows128_silu, all on the row-major merged weight
             for layer in self.model.layers:

@@ -233,11 +233,8 @@ _ROWS32_MAX = 32
 # At 33-128 token rows the same projections, and the merged w1|w3 with SiLU-mul, go to
 # delta_gemm_rows128 (us, against hipBLASLt; 64 rows: DeepSeek-R1-Distill-Qwen-1.5B w2 9.8 vs 25.4, wo
 # 4.9 vs 7.5, w1|w3 18.2 vs 18.7 and a 5 us SiLU-mul; 128 rows: Qwen2.5-14B w2 34.9 vs 73.9, wo 18.9 vs
-# 32.1, w1|w3 65-73 vs 73 and 5).  It stays on hipBLASLt where that is faster: past 64 rows most square
-# weights (see _rows128_to_norm) and gate/up launches of more than 256 blocks of 64 columns, a second pass over the CUs (Qwen2.5-7B w1|w3: 80-89
-# vs 72); wqkv and most lm_heads too, whose consumers sum no partials (see _rows128_head).
+# 32.1, w1|w3 65-73 vs 73 and 5), where it is the faster one:
 _ROWS128_MAX = 128
-_ROWS128_GLU_MAX = 64 * 256
 
 
 def _rows128_to_norm(rows: int, N: int, Kd: int) -> bool:
@@ -250,12 +247,36 @@ def _rows128_to_norm(rows: int, N: int, Kd: int) -> bool:
     return rows <= _ROWS128_MAX and (N * Kd >= 24 << 20 or (Kd >= 8192 and N * Kd >= 12 << 20))
 
 
+def _rows128_gate_up(rows: int, inter: int, dim: int) -> bool:
+    """The merged w1|w3 with SiLU-mul: one block per 64 columns of inter, so past half the chip's 256 CUs and short
+    of a block for each of them (us, against the faster of hipBLASLt's two layouts and a SiLU-mul; 64 rows: inter
+    8192 1.06-1.24 times as long, 8960 0.83-0.93, 14336 0.91-1.0, 16384 0.83-1.12; 128 rows: 8960 0.93 over
+    many layers but 1.01-1.07 while one layer's weights stay cached, 9728 0.76-1.04, 14336 0.7-0.99, 16384
+    0.76-1.11).  Past 256 blocks, up to 64 rows run two blocks of 32 columns to a CU (18944 0.86-0.96); more rows
+    take a second pass over the CUs (1.11-1.23)."""
+    if inter % 16 or dim % 64 or not _ROWS32_MAX < rows <= _ROWS128_MAX:
+        return False
+    blocks = (inter + 63) // 64
+    if rows <= 64:
+        return 128 < blocks <= 240 or blocks > 256
+    return 144 <= blocks <= 240
+
+
 def _rows128_head(rows: int, N: int, Kd: int) -> bool:
     """A wide lm_head of few features, unsplit (wqkv and other lm_heads stay on hipBLASLt: 14B wqkv unsplit 40 vs 33
     us, 8B lm_head of 4096 features 212 vs 211).  940 blocks of 128 columns are nearly four passes over the CUs, so
     the last one matters little: 0.52-1.03 of hipBLASLt for 120064-256000 columns and 1024-2048 features;
     32768 and 50304 columns 1.0-1.36, 512 features up to 1.33."""
     return _ROWS32_MAX < rows <= 64 and N >= 120000 and 1024 <= Kd <= 2048 and K.gemm_rows128_splits(rows, N, Kd) == 1
+
+
+def row_major_gate_up(batch: int, inter: int, dim: int) -> bool:
+    """Whether an engine whose decode steps have ``batch`` rows stores w1|w3 row-major (``w13``): where one of the
+    fused kernels reads it there.  Otherwise it stays transposed (``w13_t``): at 65-128 rows hipBLASLt takes 1.0-1.05
+    times as long for ``x @ w13.T`` at inter 18944.  Prompt steps run on hipBLASLt in either layout and are mostly
+    faster on the row-major one (129-8192 tokens: Llama-3-8B 0.85-0.95 of the transposed one's time, 14B 0.91-1.07,
+    7B 0.86-1.10, 1.5B 0.77-1.02; slower at 129 and 1024 tokens for 7B, 512 and 1024 for 14B)."""
+    return batch <= _ROWS32_MAX or _rows128_gate_up(batch, inter, dim)
 
 
 def dense_to_norm(x: Tensor, layer: nn.Linear):
@@ -363,8 +384,8 @@ class FeedForward(nn.Module):
     """SwiGLU FFN.  ``w1`` and ``w3`` live in one weight stored transposed, ``w13_t``
     ``[dim, 2 * inter]``, so the gate and up projections are one GEMM ``x @ w13_t``: at
     32-row decode batches hipBLASLt streams this layout at ~5.2 TB/s against ~4.4 TB/s for
-    ``x @ w13.T``.  An engine set up for at most 128 rows per step re-lays it out row-major
-    (``w13`` ``[2 * inter, dim]``, ``use_row_major_w13``): ``delta_gemm_skinny`` streams it faster
+    ``x @ w13.T``.  An engine whose steps run one of the fused kernels (``row_major_gate_up``) re-lays it out
+    row-major (``w13`` ``[2 * inter, dim]``, ``use_row_major_w13``): ``delta_gemm_skinny`` streams it faster
     still at <= 8 rows (Qwen2.5-7B, 4 rows: 41 vs 53 us) and ``delta_gemm_rows32_silu`` /
     ``delta_gemm_rows128_silu`` fuse the SiLU-mul into the GEMM at 9-32 and 33-128 rows.
     Checkpoints with separate ``w1`` / ``w3`` (the reference's names, ``[inter, dim]`` each) are
@@ -415,8 +436,7 @@ class FeedForward(nn.Module):
                 return dense_to_norm(K.gemm_skinny_silu(x, self.w13), self.w2)
             if rows <= _ROWS32_MAX:
                 return dense_to_norm(K.gemm_rows32_silu(x, self.w13), self.w2)
-        if hasattr(self, "w13") and _ROWS32_MAX < rows <= _ROWS128_MAX and self.inter % 16 == 0 \
-                and (rows <= 64 or self.inter <= _ROWS128_GLU_MAX) and K.gemm_rows128_ok(x, self.w13):
+        if hasattr(self, "w13") and _rows128_gate_up(rows, self.inter, x.shape[-1]) and K.gemm_rows128_ok(x, self.w13):
             return dense_to_norm(K.gemm_rows128_silu(x, self.w13), self.w2)
         return dense_to_norm(K.silu_mul(self._gate_up(x)), self.w2)
 

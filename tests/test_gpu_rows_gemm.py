@@ -66,12 +66,16 @@ def test_gemm_rows128_silu_matches_gemm_then_silu_mul(dtype, M, inter, Kd):
     assert (got != ref).float().mean().item() < 0.02  # and few of them do
 
 
-def test_ffn_at_33_to_128_rows_matches_the_library_path():
+def test_ffn_at_33_to_128_rows_matches_the_library_path(monkeypatch):
     """The fused FFN on the row-major weight (kernel, partials or output) against the library GEMMs
     and delta_silu_mul, a strided x included, which keeps the library's path."""
     cfg = ModelArgs.from_name("tiny-test")
+    cfg.intermediate_size = 9216
     with torch.device(DEV):
         ff = FeedForward(cfg).to(torch.bfloat16)
+    fused = []
+    silu = K.gemm_rows128_silu
+    monkeypatch.setattr(K, "gemm_rows128_silu", lambda x, w: (fused.append(x.shape[1]), silu(x, w))[1])
     with torch.inference_mode():
         gen = torch.Generator(device=DEV).manual_seed(3)
         for p in ff.parameters():
@@ -86,6 +90,7 @@ def test_ffn_at_33_to_128_rows_matches_the_library_path():
                 y = (y.sum(0) if y.dtype == torch.float32 else y.float()).view(rows, 512)
                 # both round silu(g) * u and the output to bf16: a few ulps of the row's magnitude
                 assert (y - ref).abs().max().item() <= 4 * 2 ** -8 * ref.abs().max().item()
+    assert fused == [33, 64, 65, 128]
 
 
 @torch.inference_mode()

@@ -288,3 +288,17 @@ def test_norm_projection_kernel_past_64_rows_needs_long_k_or_a_large_weight():
         assert _rows128_to_norm(64, dim, dim) and not _rows128_to_norm(65, dim, dim)
     assert _rows128_to_norm(65, 5120, 5120) and not _rows128_to_norm(96, 1024, 8192)
     assert not _rows128_to_norm(32, 4096, 14336) and not _rows128_to_norm(129, 4096, 14336)
+
+
+def test_gate_up_layout_follows_the_kernel_the_steps_run():
+    """w1|w3 is row-major exactly where a fused gate/up kernel reads it at the engine's batch: engines of 65-128 rows
+    whose gate/up stays on hipBLASLt (inter 18944, 8960) keep the transposed weight."""
+    from delta_amd.model import _rows128_gate_up, row_major_gate_up
+    for name, (inter, dim) in TABLE.items():
+        for batch in (1, 8, 32):
+            assert row_major_gate_up(batch, inter, dim)
+        for batch in (33, 64, 65, 128, 129):
+            want = batch <= 64 or (batch <= 128 and name in ("llama-3-8b", "Qwen2.5-14b"))
+            assert row_major_gate_up(batch, inter, dim) is want and _rows128_gate_up(batch, inter, dim) is want
+    for inter in (1024, 8192, 16384):
+        assert not any(_rows128_gate_up(r, inter, 4096) for r in (33, 64, 65, 128))
