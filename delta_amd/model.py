@@ -218,7 +218,8 @@ def dense(x: Tensor, layer: nn.Linear) -> Tensor:
         rows = x.numel() // x.shape[-1]
         if rows <= _SKINNY_ROWS_ANY or w.numel() * w.element_size() <= _SKINNY_MAX_WEIGHT_BYTES:
             return K.gemm_skinny(x, w, layer.bias)
-    elif _rows128_head(x.numel() // max(x.shape[-1], 1), *w.shape) and K.gemm_rows128_ok(x, w):
+    elif _rows128_head(x.numel() // max(x.shape[-1], 1), *w.shape) and K.gemm_rows128_ok(x, w) \
+            and not _own_forward(layer):
         return K.gemm_rows128(x, w, layer.bias)
     return layer(x)
 
@@ -235,6 +236,17 @@ _ROWS32_MAX = 32
 # 4.9 vs 7.5, w1|w3 18.2 vs 18.7 and a 5 us SiLU-mul; 128 rows: Qwen2.5-14B w2 34.9 vs 73.9, wo 18.9 vs
 # 32.1, w1|w3 65-73 vs 73 and 5), where it is the faster one:
 _ROWS128_MAX = 128
+
+
+def _own_forward(layer: nn.Linear) -> bool:
+    """Whether calling ``layer`` does more than ``F.linear`` on its weight and bias, which a kernel would pass by: a
+    subclass or wrapped forward, hooks, a bias that is trained or not as the kernel reads it."""
+    b = layer.bias
+    return (type(layer).forward is not nn.Linear.forward or "forward" in vars(layer) or bool(layer._forward_hooks)
+            or bool(layer._forward_pre_hooks) or bool(layer._backward_hooks) or bool(layer._backward_pre_hooks)
+            or nn.modules.module._has_any_global_hook()
+            or (b is not None and (not b.is_contiguous() or b.dtype != layer.weight.dtype
+                                   or (torch.is_grad_enabled() and b.requires_grad))))
 
 
 def _rows128_to_norm(rows: int, N: int, Kd: int) -> bool:
@@ -287,7 +299,7 @@ def dense_to_norm(x: Tensor, layer: nn.Linear):
     if rows > _SKINNY_ROWS_ANY and rows <= _ROWS32_MAX and K.gemm_skinny_ok(x, w) and w.shape[0] % 64 == 0:
         r = K.gemm_rows32(x, w, layer.bias)
         return r if r.dtype == torch.float32 else r.view(*x.shape[:-1], w.shape[0])
-    if _rows128_to_norm(rows, *w.shape) and K.gemm_rows128_ok(x, w):
+    if _rows128_to_norm(rows, *w.shape) and K.gemm_rows128_ok(x, w) and not _own_forward(layer):
         r = K.gemm_rows128(x, w, layer.bias)
         return r if r.dtype == torch.float32 else r.view(*x.shape[:-1], w.shape[0])
     return dense(x, layer)

@@ -130,6 +130,29 @@ def test_dense_to_norm_form_and_values(N, Kd, partial_rows):
             assert torch.all((y[0].float() - ref).abs() <= 2 ** -8 * ref.abs() + 1e-5 * mag + 1e-6)
 
 
+def test_a_layer_with_a_forward_of_its_own_is_called():
+    """Hooks, a subclass' or an instance's forward and a trained bias act at 33-128 rows as at any other."""
+    class Doubled(torch.nn.Linear):
+        def forward(self, x):
+            return 2 * super().forward(x)
+
+    x = torch.randn(1, 40, 256, device=DEV).bfloat16()
+    make = lambda cls=torch.nn.Linear: cls(256, 128, device=DEV, dtype=torch.bfloat16).requires_grad_(False)
+    assert not model._own_forward(make())
+    hooked, wrapped, trained = make(), make(), make()
+    seen = []
+    hooked.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+    model.dense_to_norm(x, hooked)
+    assert seen == [(1, 40, 128)]
+    doubled = make(Doubled)
+    assert torch.equal(model.dense_to_norm(x, doubled), 2 * torch.nn.functional.linear(x, doubled.weight, doubled.bias))
+    wrapped.forward = lambda t: t
+    assert model.dense_to_norm(x, wrapped) is x
+    trained.bias.requires_grad_(True)
+    model.dense_to_norm(x, trained).float().sum().backward()
+    assert torch.all(trained.bias.grad == 40)
+
+
 def test_gemm_rows128_errors():
     x = torch.zeros(33, 64, dtype=torch.bfloat16, device=DEV)
     w = torch.zeros(64, 64, dtype=torch.bfloat16, device=DEV)
