@@ -47,6 +47,10 @@ inline int merge_groups(int nsplit) {
   return n < 1 ? 1 : (n > kMergeGroups ? kMergeGroups : n);
 }
 
+// Block x of a head-major split launch: unit x (row x / nsplit, split x % nsplit) with the kv head on y, or,
+// kSplitMajor, all (row, kv head) pairs' first splits, then their second ones (see decode_plan).
+enum Numbering { kPacked = 0, kRowMajor = 1, kSplitMajor = 2 };
+
 struct DecodeArgs {
   const uint16_t *q;
   int64_t q_stride_b, q_stride_h;
@@ -69,7 +73,7 @@ struct DecodeArgs {
   int batch, hq, hkv, nsplit;
   int chunk;        // pages per work unit (split launches)
   int hb;           // kv heads per block (hkv: page-major, 1: head-major)
-  int direct;       // split launch whose block x is unit (row x / nsplit, split x % nsplit)
+  int direct;       // split launch whose blocks map to units directly (Numbering)
   int bal_w;        // unsplit head-major launch over more (row, kv head) blocks than CUs: rows per
                     // round of the balanced row order (balanced_row); 0 = block y takes row y
   float sm_scale;
@@ -355,7 +359,17 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
   const int hb = a.hb;
   const int R = nw / hb;  // waves per kv head
   // Head group: blockIdx.y of a split launch (blockIdx.x = work unit), blockIdx.x otherwise.
-  const int head0 = (a.nsplit > 1 ? (int)blockIdx.y : (int)blockIdx.x) * hb;
+  int head0 = (a.nsplit > 1 ? (int)blockIdx.y : (int)blockIdx.x) * hb;
+  int unit = blockIdx.x;
+  if (a.direct == kSplitMajor) {
+    // Block x: split x / pairs of a (row, kv head) pair, the pairs one further from split to split.
+    const int pairs = a.batch * a.hkv;
+    const int split = unit / pairs;
+    int j = unit - split * pairs + split % pairs;
+    j -= j >= pairs ? pairs : 0;
+    head0 = uniform(j % a.hkv);
+    unit = j / a.hkv * a.nsplit + split;
+  }
   const int wave = uniform(threadIdx.x >> 6);
   const int h = head0 + wave % hb;
   const int rslot = wave / hb;
@@ -365,7 +379,6 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
 
   int b, split = 0, nu = 1, j0 = 0, j1;
   RowInfo ri;
-  const int unit = blockIdx.x;
   if (a.nsplit > 1) {
     if (a.direct) {
       // Every row owns nsplit block slots: the row is known from the block index, so its bounds,
@@ -916,7 +929,7 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
     const int g = WITH_V ? (idx / kHeadDim) % G : idx % G;
     const int dd = WITH_V ? idx % kHeadDim : 0;
     float M = -INFINITY, L = 0.f, A = 0.f;
-    // R waves per head unrolled (head-major launches: 16, or 4 when unsplit), so all the LDS
+    // R waves per head unrolled (head-major launches: 16, 8 or 4), so all the LDS
     // reads issue together (same sums in the same order as the loop below).
     auto unrolled = [&](auto rw) {
       constexpr int RW = decltype(rw)::value;
@@ -940,6 +953,8 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
     };
     if (kOwnMerge && R == kMaxWaves) {
       unrolled(std::integral_constant<int, kMaxWaves>());
+    } else if (kOwnMerge && R == 8) {
+      unrolled(std::integral_constant<int, 8>());
     } else if (kOwnMerge && R == kHeadMajorWaves) {
       unrolled(std::integral_constant<int, kHeadMajorWaves>());
     } else {
@@ -1136,7 +1151,9 @@ enum Mode { kAttn = 0, kAttnDump = 1, kScoreOnly = 2, kAttnSubset = 3, kScoreTok
 
 template <int DT, int G>
 void launch_split(const DecodeArgs &a, int waves, int mode, hipStream_t stream) {
-  dim3 grid = a.nsplit > 1 ? dim3(a.batch * a.nsplit, a.hkv / a.hb) : dim3(a.hkv / a.hb, a.batch);
+  dim3 grid = a.direct == kSplitMajor ? dim3(a.batch * a.nsplit * a.hkv)
+              : a.nsplit > 1          ? dim3(a.batch * a.nsplit, a.hkv / a.hb)
+                                      : dim3(a.hkv / a.hb, a.batch);
   dim3 block(64 * waves);
   const bool rope = a.k_new != nullptr;
   const size_t merge = (size_t)waves * G * (2 + kHeadDim) * sizeof(float);
@@ -1263,7 +1280,8 @@ int device_cus() {
 constexpr int64_t kHeadMajorPageHeads = 262144;
 constexpr int kMaxChunk = 128;
 
-void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int *waves, int *hb, int *chunk) {
+void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int *waves, int *hb, int *chunk,
+                 int *direct) {
   const bool unsplit = (int64_t)batch * hkv >= kHeadMajorPairs &&
                        (int64_t)batch * hkv * max_pages <= kHeadMajorPageHeads;
   const bool small = !dump && (int64_t)batch * hkv < kHeadMajorPairs;
@@ -1304,11 +1322,7 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
   // us; at config 4, 16 -> 64 splits, the merge's 4x partials cost more than the block merge
   // saves: 13.6 -> 14.2 us).  Others keep 16 waves (the config-4 full attention, 128-page units:
   // with 4 waves its full-cache engine step ran 5.4-5.6 -> 5.9-6.0 ms, though a launch timed alone
-  // was unchanged).  One-wave units of up to 16 pages and 8-wave units of 64 were measured over 12
-  // (rows, kv heads), 40-2100 max_pages and rows of 10-100 % of it: faster at most of them (50 rows of
-  // 133 pages, 2 kv heads: 32.6 -> 25.4 us), but 1.1-1.4 times as long at a third (rows of 13 pages
-  // under max_pages 133: 12.9 -> 16.1; 64 rows of 66 under 264: 23.2 -> 32.1; 8 rows of 264, 8 kv heads:
-  // 29.8 -> 36.1), and max_pages says nothing about the rows' lengths, so no rule on it can tell.
+  // was unchanged).
   if (small && ceil_div(ch, (int64_t)kHeadMajorWaves) <= 8) {
     R = kHeadMajorWaves;
     if (ns > 1 && ns * kHeadMajorWaves <= 16 && ns * kHeadMajorWaves <= max_pages) {
@@ -1316,6 +1330,26 @@ void decode_plan(int batch, int hkv, int max_pages, bool dump, int *nsplit, int 
       ch = ceil_div(max_pages, ns);
       R = 1;
     }
+  }
+  *direct = ns > 1 && h == 1 ? kRowMajor : kPacked;
+  const int64_t pairs = (int64_t)batch * hkv, page_heads = pairs * max_pages;
+  if (small && ceil_div(ch, (int64_t)kHeadMajorWaves) > 8 && pairs >= 64 && page_heads >= 16000 && page_heads <= 600000) {
+    // Longer units (the full attention of small batches): 8-wave units, about 1000 of them, of 32-96 pages,
+    // numbered split by split.  Numbered row by row, split s of every row lands on XCD s % 8 where their
+    // number is a multiple of 8 (blocks go to the XCDs round robin), and rows far below max_pages, which is
+    // often a slot's size, leave XCDs idle; finer units alone then made a third of the shapes slower (64 rows of
+    // 66 pages under max_pages 264, 2 kv heads: 23.2 us with units of 88 pages, 32.1 with 64, 19.3 with 32
+    // split by split).  Against the 16-wave units of up to 128 pages, over 1002 calls (17 pairs of rows and kv
+    // heads, max_pages 69-4100, rows of 10-100 % of it and ragged): 0.86 of the time on average, 0.38-1.07, five
+    // calls of ragged rows over 1.05.  Not taken: fewer pairs (32-63: up to 1.17), less to read (8 rows of up to 200
+    // pages, 8 kv heads: up to 1.15), and more than 600000 page-heads, which were not measured and would need a third
+    // more partials.
+    const int64_t fill = ceil_div(1000, pairs), most = max_pages / 32, least = ceil_div(max_pages, 96);
+    ns = fill < most ? fill : most;
+    ns = ns > least ? ns : least;
+    ch = ceil_div(max_pages, ns);
+    R = 8;
+    *direct = kSplitMajor;
   }
   *nsplit = (int)ns;
   *waves = h * R;
@@ -1340,9 +1374,9 @@ bool plan_tokmax_fits(int batch, int hkv, int G, int max_pages, bool rope) {
 }
 
 int decode_num_splits(int batch, int hkv, int max_pages) {
-  int ns, w, hb, ch, ns_dump;
-  decode_plan(batch, hkv, max_pages, false, &ns, &w, &hb, &ch);
-  decode_plan(batch, hkv, max_pages, true, &ns_dump, &w, &hb, &ch);
+  int ns, w, hb, ch, dir, ns_dump;
+  decode_plan(batch, hkv, max_pages, false, &ns, &w, &hb, &ch, &dir);
+  decode_plan(batch, hkv, max_pages, true, &ns_dump, &w, &hb, &ch, &dir);
   return ns > ns_dump ? ns : ns_dump;
 }
 
@@ -1421,19 +1455,17 @@ int run_decode(const void *q, int64_t q_stride_b, int64_t q_stride_h, const void
   a.hq = hq;
   a.hkv = hkv;
   int waves;
-  decode_plan(batch, hkv, max_pages, dump != nullptr, &a.nsplit, &waves, &a.hb, &a.chunk);
+  decode_plan(batch, hkv, max_pages, dump != nullptr, &a.nsplit, &waves, &a.hb, &a.chunk, &a.direct);
   if (tokmax) {  // head-major, unsplit: each block ends with its head's final lse
     // 4 waves (one per SIMD), as the other unsplit head-major launches: config-3 planner
     // 176.1 -> 169.7 us and K-only scorer 92.2 -> 88.5 us against 16 waves (8 waves: 173.3 /
     // 91.7).
     a.nsplit = 1;
     a.hb = 1;
+    a.direct = kPacked;
     waves = kHeadMajorWaves;
     a.chunk = max_pages;
   }
-  // Head-major split launches (small batches: fewer than 256 (row, kv head) pairs) map blocks to
-  // units directly; page-major ones pack a ragged batch's units at the front of the grid.
-  a.direct = a.nsplit > 1 && a.hb == 1;
   // Unsplit head-major launches with more blocks than CUs deal ragged rows to CUs evenly.
   const int cus = device_cus();
   a.bal_w = (a.nsplit == 1 && a.hb == 1 && (int64_t)batch * hkv > cus && batch <= kBalanceMaxRows &&

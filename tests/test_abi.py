@@ -105,10 +105,11 @@ def test_prefill_rows_workspace_is_bounded(lib):
 
 
 def test_small_attention_plans(lib):
-    """Attention launches of 32-255 pairs: about 256 blocks, units of at most 128 pages.  Finer units were
-    faster for full rows and slower for rows far below max_pages, which the plan cannot see.  (The query
-    is the larger of this plan and the dump launch's, here the first.)"""
-    for (batch, hkv, pages), splits in {(100, 2, 69): 2, (60, 4, 69): 2, (100, 2, 1153): 10, (60, 4, 2100): 17}.items():
+    """Attention launches of 64-255 pairs and 16000-600000 page-heads: about 1000 units of 32-96 pages; outside,
+    about 256 blocks and units of at most 128 pages.  (The query is the larger of this plan and the dump
+    launch's.)"""
+    for (batch, hkv, pages), splits in {(100, 2, 69): 2, (64, 2, 517): 8, (64, 2, 1153): 13, (100, 2, 2100): 22,
+                                        (60, 4, 2500): 27, (60, 4, 2501): 20, (31, 2, 2100): 17}.items():
         assert lib.delta_decode_num_splits(batch, hkv, pages) == max(splits, _dump_splits(batch, hkv, pages))
 
 
