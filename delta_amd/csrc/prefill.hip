@@ -78,8 +78,10 @@ constexpr int kTileB = kKvStep * 256;  // bytes of a step's K (or V) tile: 64 ro
 //   kByRow, more rows: a row's last tile first, then the next row.  What runs together shares few rows' K
 //     and V in the L2 (16 prompts of 512, 8 kv heads 79.6 / 71.5; 32 of 64-256 40.8 / 36.4; 64 of 128
 //     66.0 / 52.3).
-//   kBySlot, one row or no more slots than the CUs hold at once: nothing to order, no search in front (100
-//     prompts of 30, 2 kv heads 11.8 / 12.2 by row).
+//   kBySlot, one row or a CU for every slot: nothing to order, no search in front (100 prompts of 30, 2 kv
+//     heads 11.8 / 12.2 by row).  With a second block on some CUs the order matters for rows of many tiles (4
+//     prompts of 331 at 1331 tokens, 4 kv heads, 336 slots: 44.9 / 40.0 by tile), not for few (20 of 60, 320
+//     slots: 11.1 / 11.9 by row).
 enum BlockOrder { kBySlot = 0, kByRow = 1, kByTile = 2 };
 constexpr int kByTileRows = 12;
 
@@ -153,26 +155,42 @@ __device__ __forceinline__ float halves_sum(float v) {
   return __uint_as_float(x[0]) + __uint_as_float(x[1]);
 }
 
-// Row and tile (BT query tokens) of block u of a kv head; false past the last one.  Only the device knows
-// the rows' lengths, so the grid has batch * row_tiles slots.
+// A row's CSR bounds and last page length.
+struct RowBounds {
+  int q0, q1, kv0, kv1, last;
+};
+__device__ __forceinline__ RowBounds row_bounds(const PrefillArgs &a, int r) {
+  return r < a.batch ? RowBounds{a.qo_indptr[r], a.qo_indptr[r + 1], a.kv_indptr[r], a.kv_indptr[r + 1], a.last_page_len[r]}
+                     : RowBounds{0, 0, 0, 0, 0};
+}
+__device__ __forceinline__ RowBounds bounds_of_lane(const RowBounds &x, int l) {
+  return RowBounds{__builtin_amdgcn_readlane(x.q0, l), __builtin_amdgcn_readlane(x.q1, l),
+                   __builtin_amdgcn_readlane(x.kv0, l), __builtin_amdgcn_readlane(x.kv1, l),
+                   __builtin_amdgcn_readlane(x.last, l)};
+}
+
+// Row, with its bounds, and tile (BT query tokens) of block u of a kv head; false past the last one.  Only the
+// device knows the rows' lengths, so the grid has batch * row_tiles slots.  Every lane loads a row's bounds, so
+// that the row found costs no second round trip.
 template <int BT>
-__device__ __forceinline__ bool find_tile(const PrefillArgs &a, int u, int lane, int *row, int *tile) {
-  auto tiles_of = [&](int r) {
-    if (r >= a.batch) return 0;
-    const int qn = a.qo_indptr[r + 1] - a.qo_indptr[r];
+__device__ __forceinline__ bool find_tile(const PrefillArgs &a, int u, int lane, RowBounds *row, int *tile) {
+  auto tiles_of = [&](const RowBounds &x) {
+    const int qn = x.q1 - x.q0;
     if (qn <= 0 || (a.skip_single && qn == 1)) return 0;
     const int n = (qn + BT - 1) / BT;
     return n < a.row_tiles ? n : a.row_tiles;
   };
   if (a.order == kBySlot) {
-    *row = u / a.row_tiles;
-    *tile = a.row_tiles - 1 - (u - *row * a.row_tiles);
-    return *row < a.batch && *tile < tiles_of(*row);
+    const int r = u / a.row_tiles;
+    *row = row_bounds(a, r);
+    *tile = a.row_tiles - 1 - (u - r * a.row_tiles);
+    return *tile < tiles_of(*row);
   }
   if (a.order == kByTile) {  // batch <= 64, row_tiles <= 32 * 64
     // Lane l counts the blocks from tile t_l on, sum over the rows of max(0, n_r - t_l), for 64 t at
     // once (more tiles: coarse, then fine).
-    const int n = tiles_of(lane);
+    const RowBounds mine = row_bounds(a, lane);
+    const int n = tiles_of(mine);
     auto blocks_from = [&](int t) {
       int s = 0;
       for (int r = 0; r < a.batch; ++r) {
@@ -198,14 +216,15 @@ __device__ __forceinline__ bool find_tile(const PrefillArgs &a, int u, int lane,
     // order would give an XCD all tiles of the same rows.
     const uint64_t has = __ballot(n > t);
     const int i = (u - above + t) % __popcll(has);
-    const bool mine = n > t && __popcll(has & ((1ull << lane) - 1)) == i;
-    *row = __builtin_ctzll(__ballot(mine));
+    const uint64_t it = __ballot(n > t && __popcll(has & ((1ull << lane) - 1)) == i);
+    *row = bounds_of_lane(mine, __builtin_ctzll(it));
     *tile = t;
     return true;
   }
   int base = 0;
   for (int r0 = 0; r0 < a.batch; r0 += 64) {
-    const int n = tiles_of(r0 + lane);
+    const RowBounds mine = row_bounds(a, r0 + lane);
+    const int n = tiles_of(mine);
     int incl = n;
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
@@ -215,7 +234,7 @@ __device__ __forceinline__ bool find_tile(const PrefillArgs &a, int u, int lane,
     const uint64_t m = __ballot(base + incl > u);
     if (m != 0) {
       const int l = __builtin_ctzll(m);
-      *row = r0 + l;
+      *row = bounds_of_lane(mine, l);
       *tile = base + __builtin_amdgcn_readlane(incl, l) - 1 - u;
       return true;
     }
@@ -241,23 +260,25 @@ __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int hl = lane >> 5, n = lane & 31;
   const int h = blockIdx.x;
-  int b, tile;
-  if (!find_tile<BT>(a, (int)(blockIdx.z * gridDim.y + blockIdx.y), lane, &b, &tile)) return;  // whole block
-  const int64_t q0 = a.qo_indptr[b], q1 = a.qo_indptr[b + 1];
-  const int qn = (int)(q1 - q0);
+  RowBounds row;
+  int tile;
+  if (!find_tile<BT>(a, (int)(blockIdx.z * gridDim.y + blockIdx.y), lane, &row, &tile)) return;  // whole block
+  const int64_t q0 = row.q0;
+  const int qn = row.q1 - row.q0;
   const int btok0 = tile * BT;
   // The wave's first query token, read as a scalar: the compiler cannot see that wave (from the
   // thread index) is uniform, and with tok0 scalar the wave's step count and its diagonal test
-  // (full / masked step) become scalar branches (8192-token prompt 594 -> 569-585 us).
+  // (full / masked step) become scalar branches (8192-token prompt 594 -> 569-585 us in the kernel that
+  // staged K and V through registers).
   const int tok0 = __builtin_amdgcn_readfirstlane(btok0 + wave * TW);
 
   // Row's pages and length (indptr entries clamped as in the decode kernels).
   const int64_t ilen = a.kv_indices_len;
-  int64_t p0 = a.kv_indptr[b], p1 = a.kv_indptr[b + 1];
+  int64_t p0 = row.kv0, p1 = row.kv1;
   p0 = p0 < 0 ? 0 : (p0 > ilen ? ilen : p0);
   p1 = p1 < p0 ? p0 : (p1 > ilen ? ilen : p1);
   const int np = (int)(p1 - p0);
-  int lp = a.last_page_len[b];
+  int lp = row.last;
   lp = lp < 0 ? 0 : (lp > kPageSize ? kPageSize : lp);
   const int kv_len = np > 0 ? (np - 1) * kPageSize + lp : 0;
 
@@ -387,8 +408,9 @@ __global__ void __launch_bounds__(PW * 64, 2) paged_prefill_kernel(PrefillArgs a
 #pragma unroll
       for (int sb = 0; sb < kSub; ++sb) kq[s][sb] = kfrag(sb, s);
     __builtin_amdgcn_sched_barrier(0);
-    // Raised wave priority over each MFMA run: of the SIMD's two waves, the one with MFMAs
-    // to issue goes first, which pushes the other into its softmax meanwhile (8192 tokens 569 -> 517 us).
+    // Raised wave priority over each MFMA run: of the SIMD's two waves, the one with MFMAs to issue goes
+    // first, which pushes the other into its softmax meanwhile (8192 tokens 542 -> 512 us; 300 and 2048 tokens,
+    // in 4-wave blocks, the same within 1-2 %).
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int ks = 0; ks < 8; ++ks) {
@@ -557,14 +579,14 @@ bool wide_blocks(const PrefillArgs &a, int bt4, int max_qo) {
   // of 20, 4 kv heads of 7 (240 / 480 blocks) 10.2 / 12.6 us; 100 of 30, 2 of 6 (200 / 400) 10.9 / 11.8.
   const int64_t blocks = (int64_t)a.batch * a.hkv;
   if (max_qo > bt4 && max_qo <= 2 * bt4 && blocks <= 256 && 2 * blocks > 256) return true;
-  // Prompts continued over at least three times as many cached tokens, whose blocks all sweep about as far,
-  // and more 4-wave blocks than one to a CU: 1500 tokens at 16 k (376 blocks) 426 / 464 us, 2048 at 8 k (512)
-  // 284 / 298, 8 of 256 at 4 k (512) 139 / 149; but 1024 at 8 k (256) 222 / 195, 3000 at 8 k (2.7 times) 482 /
-  // 479, 2048 at 4 k (twice) 172 / 172.
+  // Prompts continued over at least 3.5 times as many cached tokens, whose blocks all sweep about as far, and
+  // well more 4-wave blocks than one to a CU: 1500 tokens at 16 k (376 blocks) 426 / 464 us, 2048 at 8 k (512)
+  // 284 / 298, 8 of 256 at 4 k (512) 139 / 149; but 1024 at 8 k (256) 222 / 195, 4 of 331 at 1 k (331, three
+  // times; with RoPE + append) 49.4 / 47.5, 3000 at 8 k (2.7 times) 482 / 479, 2048 at 4 k (twice) 172 / 172.
   if (a.num_tokens < 0) return false;
   const int64_t tokens = a.num_tokens - a.decode_rows;
   const int64_t cached = (a.kv_indices_len - a.decode_pages) * kPageSize - tokens;
-  return cached >= 3 * tokens && tokens * a.hkv >= 300 * (int64_t)bt4;
+  return 2 * cached >= 7 * tokens && tokens * a.hkv >= 350 * (int64_t)bt4;
 }
 
 template <int DT, int G>
@@ -573,7 +595,7 @@ void launch_prefill_g(PrefillArgs a, int max_qo, hipStream_t stream) {
   const int bt = 32 / G * (wide ? 8 : 4);
   a.row_tiles = (int)ceil_div(max_qo, bt);
   const int64_t slots = (int64_t)a.batch * a.row_tiles;
-  a.order = a.batch == 1 || slots * a.hkv <= (wide ? 256 : 512) ? kBySlot
+  a.order = a.batch == 1 || slots * a.hkv <= (a.row_tiles <= 4 ? 512 : 256) ? kBySlot
             : a.batch <= kByTileRows && a.row_tiles <= 32 * 64  ? kByTile
                                                                 : kByRow;
   // Tiles of that many tokens over that many rows, at most: what is launched past the last one only exits, but
