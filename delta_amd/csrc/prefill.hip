@@ -160,8 +160,8 @@ struct RowBounds {
   int q0, q1, kv0, kv1, last;
 };
 __device__ __forceinline__ RowBounds row_bounds(const PrefillArgs &a, int r) {
-  return r < a.batch ? RowBounds{a.qo_indptr[r], a.qo_indptr[r + 1], a.kv_indptr[r], a.kv_indptr[r + 1], a.last_page_len[r]}
-                     : RowBounds{0, 0, 0, 0, 0};
+  if (r >= a.batch) return RowBounds{0, 0, 0, 0, 0};
+  return RowBounds{a.qo_indptr[r], a.qo_indptr[r + 1], a.kv_indptr[r], a.kv_indptr[r + 1], a.last_page_len[r]};
 }
 __device__ __forceinline__ RowBounds bounds_of_lane(const RowBounds &x, int l) {
   return RowBounds{__builtin_amdgcn_readlane(x.q0, l), __builtin_amdgcn_readlane(x.q1, l),
@@ -675,8 +675,8 @@ int run_prefill(const void *q, int64_t q_stride_t, int64_t q_stride_h, const voi
     if ((uintptr_t)workspace & 255u) return set_error(DELTA_ERR_INVALID, "%s: workspace must be 256-byte aligned", who);
     const int rc = run_decode_rows(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
                                    kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
-                                   num_kv_heads, dtype, sm_scale, decode_pages, decode_max_pages, workspace, (hipStream_t)stream,
-                                   who);
+                                   num_kv_heads, dtype, sm_scale, decode_pages, decode_max_pages, workspace,
+                                   (hipStream_t)stream, who);
     if (rc || max_qo_len == 1) return rc;
   }
   if (dtype == DELTA_BF16)
@@ -722,7 +722,8 @@ extern "C" DELTA_EXPORT int delta_paged_prefill_rows(const void *q, int64_t q_st
       (num_tokens < 0 || decode_rows < 0 || decode_rows > batch || decode_pages < 0 || decode_pages > kv_indices_len ||
        decode_max_pages < 0 || decode_max_pages > decode_pages)) {
     delta::clear_error();
-    return delta::set_error(DELTA_ERR_INVALID, "%s: num_tokens, decode_rows, decode_pages or decode_max_pages out of range", who);
+    return delta::set_error(DELTA_ERR_INVALID,
+                            "%s: num_tokens, decode_rows, decode_pages or decode_max_pages out of range", who);
   }
   return delta::run_prefill(q, q_stride_t, q_stride_h, kv_cache, num_pages, qo_indptr, kv_indptr, kv_indices,
                             kv_indices_len, kv_last_page_len, o, o_stride_t, o_stride_h, lse, batch, num_qo_heads,
