@@ -360,15 +360,16 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
   const int R = nw / hb;  // waves per kv head
   // Head group: blockIdx.y of a split launch (blockIdx.x = work unit), blockIdx.x otherwise.
   int head0 = (a.nsplit > 1 ? (int)blockIdx.y : (int)blockIdx.x) * hb;
-  int unit = blockIdx.x;
+  const int unit = blockIdx.x;
+  int b, split = 0;
   if (a.direct == kSplitMajor) {
     // Block x: split x / pairs of a (row, kv head) pair, the pairs one further from split to split.
     const int pairs = a.batch * a.hkv;
-    const int split = unit / pairs;
+    split = uniform(unit / pairs);
     int j = unit - split * pairs + split % pairs;
     j -= j >= pairs ? pairs : 0;
-    head0 = uniform(j % a.hkv);
-    unit = j / a.hkv * a.nsplit + split;
+    b = uniform(j / a.hkv);
+    head0 = uniform(j - b * a.hkv);
   }
   const int wave = uniform(threadIdx.x >> 6);
   const int h = head0 + wave % hb;
@@ -377,14 +378,16 @@ __device__ __forceinline__ void decode_split_body(const DecodeArgs &a, float *sm
   const int c = lane >> 4;
   const int t = lane & 15;
 
-  int b, split = 0, nu = 1, j0 = 0, j1;
+  int nu = 1, j0 = 0, j1;
   RowInfo ri;
   if (a.nsplit > 1) {
     if (a.direct) {
       // Every row owns nsplit block slots: the row is known from the block index, so its bounds,
       // q and page ids load with no scan before them; slots past the row's units exit.
-      b = uniform(unit / a.nsplit);
-      split = uniform(unit - b * a.nsplit);
+      if (a.direct == kRowMajor) {
+        b = uniform(unit / a.nsplit);
+        split = uniform(unit - b * a.nsplit);
+      }
       ri = row_info(a, b);
       nu = (ri.np + a.chunk - 1) / a.chunk;
       nu = nu < 1 ? 1 : (nu > a.nsplit ? a.nsplit : nu);
