@@ -131,6 +131,15 @@ def test_prefill_block_orders_match_a_row_at_a_time(lens):
         assert torch.equal(o1, o[qo[b]:qo[b + 1]]) and torch.equal(l1, lse[qo[b]:qo[b + 1]])
 
 
+def test_prefill_grid_of_more_slots_than_one_dimension_holds():
+    """max_qo_len may exceed every row: 300 rows x 188 tiles are 56400 slots, most without a block, over two grid
+    layers; the same bits as with the rows' own maximum."""
+    c = build([(40, 40)] * 250 + [(7, 90)] * 50, 28, 4, torch.bfloat16, seed=9)
+    o0, l0 = launch(c, False, 40)
+    o1, l1 = launch(c, False, 3000)
+    assert torch.equal(o0, o1) and torch.equal(l0, l1)
+
+
 @torch.inference_mode()  # as the engine captures: torch's graph state must not change mode between captures
 def test_paged_prefill_takes_the_rows_path_where_it_should():
     assert K._prefill_has_decode_rows(808, 32, 777, 32 * 300)
